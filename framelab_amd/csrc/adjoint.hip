@@ -15,6 +15,7 @@
 #include "fl_common.h"
 #include "fl_geom.h"
 #include "fl_fan.h"
+#include "fl_fan_adj.h"
 
 // Workgroups per CU the register budget is sized for (a build-time tuning
 // knob; the default is the measured optimum at 256^3).
@@ -22,6 +23,7 @@
 #define FL_EXACT_WG_PER_CU 5
 #endif
 
+// General form: one lane per pixel (fl_fan_adj_pixel).
 template <typename YT, typename XT>
 __global__ __launch_bounds__(256) void k_adj_fan(const YT* __restrict__ Y, XT* __restrict__ X, AdjGeom g)
 {
@@ -254,10 +256,9 @@ __global__ __launch_bounds__(256, FL_EXACT_WG_PER_CU) void k_adj_cone_zc(const Y
     }
 }
 
-// Per (view, cell) of a fan plan, the two quotients of the cell's line
-// chord that do not depend on the pixel (fl_chord_line2_q): the line's
-// coefficients formed exactly as fl_fan_adj_pixel forms them.
-__global__ __launch_bounds__(256) void k_fan_line_q(AdjGeom g, int nv, float2* __restrict__ out)
+// Per (view, cell) of a fan plan, the cell's line and its quotients that do
+// not depend on the pixel (Atx_fan_mf_cpu_new.cpp:50-53, find_l.cpp:28-42).
+__global__ __launch_bounds__(256) void k_fan_line_q(AdjGeom g, int nv, float4* __restrict__ out, float* __restrict__ pd)
 {
     const size_t k = (size_t)blockIdx.x * 256 + threadIdx.x;
     if (k >= (size_t)nv * g.na) return;
@@ -268,13 +269,13 @@ __global__ __launch_bounds__(256) void k_fan_line_q(AdjGeom g, int nv, float2* _
     const float Py = cd * c - sd * s;
     const float a2 = fl_absf(Px), b2 = fl_absf(Py);
     const float hx = a2 / 2, hy = b2 / 2;
-    out[k] = make_float2((hx < hy) ? 1.0f / b2 : 1.0f / a2, 1.0f / (a2 * b2));
+    out[k] = make_float4(2 * Px, 2 * Py, (hx < hy) ? 1.0f / b2 : 1.0f / a2, 0.25f * (1.0f / (a2 * b2)));
+    if (iv == 0) pd[id] = 2 * (g.SO * sd);
 }
 
-// Per (view, cell) of a fan plan: (1/dx, 1/dy, |d|) of the ray, formed as
-// fl_fan_matched_pixel forms them (zero direction components give infinite
-// reciprocals, which the slab routine never uses).
-__global__ __launch_bounds__(256) void k_fan_ray_q(FwdGeom f, int nv, float4* __restrict__ out)
+// Per (view, cell) of a fan plan: the ray's (dx, dy, 1/dx, 1/dy), formed as
+// the forward forms dx and dy, and its length.
+__global__ __launch_bounds__(256) void k_fan_ray_q(FwdGeom f, int nv, float4* __restrict__ out, float* __restrict__ len)
 {
     const size_t k = (size_t)blockIdx.x * 256 + threadIdx.x;
     if (k >= (size_t)nv * f.na) return;
@@ -285,31 +286,35 @@ __global__ __launch_bounds__(256) void k_fan_ray_q(FwdGeom f, int nv, float4* __
     const float x2 = c * f.OD - s * yd;
     const float y2 = s * f.OD + c * yd;
     const float dx = x2 - x1, dy = y2 - y1;
-    out[k] = make_float4(1.0f / dx, 1.0f / dy, sqrtf(dx * dx + dy * dy), 0.0f);
+    out[k] = make_float4(dx, dy, dx != 0.0f ? 1.0f / dx : 0.0f, dy != 0.0f ? 1.0f / dy : 0.0f);
+    len[k] = sqrtf(dx * dx + dy * dy);
 }
 
-hipError_t fl_launch_fan_ray_q(const FwdGeom& f, int nv, float4* out, hipStream_t st)
+hipError_t fl_launch_fan_ray_q(const FwdGeom& f, int nv, float4* out, float* len, hipStream_t st)
 {
     const size_t n = (size_t)nv * f.na;
     if (n == 0) return hipSuccess;
-    hipLaunchKernelGGL(k_fan_ray_q, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, f, nv, out);
+    hipLaunchKernelGGL(k_fan_ray_q, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, f, nv, out, len);
     return hipGetLastError();
 }
 
-hipError_t fl_launch_fan_line_q(const AdjGeom& g, int nv, float2* out, hipStream_t st)
+hipError_t fl_launch_fan_line_q(const AdjGeom& g, int nv, float4* out, float* pd, hipStream_t st)
 {
     const size_t n = (size_t)nv * g.na;
     if (n == 0) return hipSuccess;
-    hipLaunchKernelGGL(k_fan_line_q, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, g, nv, out);
+    hipLaunchKernelGGL(k_fan_line_q, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, g, nv, out, pd);
     return hipGetLastError();
 }
 
 template <typename YT, typename XT>
-static hipError_t launch_adj_fan_t(const void* Y, void* X, const AdjGeom& g, hipStream_t st)
+static hipError_t launch_adj_fan_t(const void* Y, void* X, const FwdGeom& f, const AdjGeom& g, hipStream_t st)
 {
     dim3 grid((g.nx + 15) / 16, (g.ny + 15) / 16, g.nt);
     if (grid.x == 0 || grid.y == 0 || grid.z == 0) return hipSuccess;
-    hipLaunchKernelGGL((k_adj_fan<YT, XT>), grid, dim3(16, 16), 0, st, (const YT*)Y, (XT*)X, g);
+    const YT* y = (const YT*)Y;
+    XT* x = (XT*)X;
+    if (!fl_launch_fan_adj_w<FanExact>(y, x, f, g, st))
+        hipLaunchKernelGGL((k_adj_fan<YT, XT>), grid, dim3(16, 16), 0, st, y, x, g);
     return hipGetLastError();
 }
 
@@ -335,9 +340,10 @@ static hipError_t launch_adj_cone_t(const void* Y, void* X, const AdjGeom& g, hi
         return hipErrorInvalidValue;                                                         \
     } while (0)
 
-hipError_t fl_launch_adj_fan(const void* Y, int yt, void* X, int xt, const AdjGeom& g, hipStream_t st)
+hipError_t fl_launch_adj_fan(const void* Y, int yt, void* X, int xt, const FwdGeom& f, const AdjGeom& g,
+                             hipStream_t st)
 {
-    FL_DISPATCH_YX(launch_adj_fan_t, yt, xt, Y, X, g, st);
+    FL_DISPATCH_YX(launch_adj_fan_t, yt, xt, Y, X, f, g, st);
 }
 
 hipError_t fl_launch_adj_cone(const void* Y, int yt, void* X, int xt, const AdjGeom& g, hipStream_t st)

@@ -22,6 +22,7 @@
 #include "../../include/framelab_hip.h"
 #include "fl_capi_internal.h"
 #include "fl_fan.h"
+#include "fl_fan_adj.h"
 #include "fl_framelet.h"
 #include "fl_framelet_dev.h"
 
@@ -34,7 +35,7 @@ struct BDesc {
     AdjGeom a;
     long long voff, soff;    // packed offsets of the problem's volume / sinogram
     int n;                   // pixels
-    int fwd0, adj0, vec0;    // first work item of each kind
+    int fwd0, vec0;          // first work item of each kind
 };
 
 struct BState {
@@ -78,6 +79,7 @@ __global__ __launch_bounds__(64) void k_bfwd(const float* __restrict__ X, float*
     }
 }
 
+// Items of the problems without the windowed form (fl_fan_adj.h).
 template <bool MATCHED>
 __global__ __launch_bounds__(64) void k_badj(const float* __restrict__ Y, float* __restrict__ X,
                                             const BDesc* __restrict__ D, const int* __restrict__ start, int P,
@@ -91,10 +93,43 @@ __global__ __launch_bounds__(64) void k_badj(const float* __restrict__ Y, float*
         const int ix = (local % tx) * 8 + (threadIdx.x & 7), iy = (local / tx) * 8 + (threadIdx.x >> 3);
         if (ix < nx && iy < ny) {
             const float* y = Y + D[p].soff;
-            const float v = MATCHED ? fl_fan_matched_pixel<float, false>(y, D[p].f, D[p].a, 0, ix, iy)
-                                    : fl_fan_adj_pixel<float, false>(y, D[p].a, 0, ix, iy);
+            const float v = MATCHED ? fl_fan_matched_pixel(y, D[p].f, D[p].a, 0, ix, iy)
+                                    : fl_fan_adj_pixel(y, D[p].a, 0, ix, iy);
             X[D[p].voff + (size_t)iy * nx + ix] = v;
         }
+    }
+}
+
+// Items of the problems with the windowed form: one 8 x 8 tile per workgroup
+// at a time, its views shared by FAN_W waves.
+template <class Kind>
+__global__ __launch_bounds__(64 * (FAN_W + 1)) void k_badj_w(const float* __restrict__ Y, float* __restrict__ X,
+                                                            const BDesc* __restrict__ D,
+                                                            const int* __restrict__ start, int P, int total)
+{
+    __shared__ union {
+        FanTileLds<2, FAN_W, fl_fan_vb(2)> s2;
+        FanTileLds<3, FAN_W, fl_fan_vb(3)> s3;
+        FanTileLds<4, FAN_W, fl_fan_vb(4)> s4;
+        FanTileLds<6, FAN_W, fl_fan_vb(6)> s6;
+    } lds;
+    for (int item = blockIdx.x; item < total; item += gridDim.x) {
+        const int p = find_problem(start, P, item);
+        const int local = item - start[p];
+        const AdjGeom& g = D[p].a;
+        const FwdGeom& f = D[p].f;
+        const int nx = f.nx, ny = f.ny, tx = (nx + 7) / 8;
+        const int ix0 = (local % tx) * 8, iy0 = (local / tx) * 8;
+        const float* y = Y + D[p].soff;
+        float v;
+        switch (g.fan_cells) {
+        case 2: v = fl_fan_adj_tile<Kind, 2, FAN_W, fl_fan_vb(2)>(y, f, g, 0, ix0, iy0, lds.s2); break;
+        case 3: v = fl_fan_adj_tile<Kind, 3, FAN_W, fl_fan_vb(3)>(y, f, g, 0, ix0, iy0, lds.s3); break;
+        case 4: v = fl_fan_adj_tile<Kind, 4, FAN_W, fl_fan_vb(4)>(y, f, g, 0, ix0, iy0, lds.s4); break;
+        default: v = fl_fan_adj_tile<Kind, 6, FAN_W, fl_fan_vb(6)>(y, f, g, 0, ix0, iy0, lds.s6); break;
+        }
+        const int lane = threadIdx.x & 63, ix = ix0 + (lane & 7), iy = iy0 + (lane >> 3);
+        if ((int)threadIdx.x >> 6 == FAN_W && ix < nx && iy < ny) X[D[p].voff + (size_t)iy * nx + ix] = v;
     }
 }
 
@@ -321,8 +356,9 @@ struct fl_batch_s {
     std::vector<BDesc> desc;
     std::vector<long long> voff, soff;   // P+1 each
     BDesc* d_desc = nullptr;
-    int *d_fstart = nullptr, *d_astart = nullptr, *d_vstart = nullptr;
-    int fwd_total = 0, adj_total = 0, vec_total = 0;
+    // first items per problem; adjoint items split by form (general, windowed)
+    int *d_fstart = nullptr, *d_astart = nullptr, *d_wstart = nullptr, *d_vstart = nullptr;
+    int fwd_total = 0, adj_total = 0, adjw_total = 0, vec_total = 0;
     int T = 64;                          // rays per forward item
     int fwd_grid = 0, adj_grid = 0, vec_grid = 0;
     // solver workspace
@@ -376,7 +412,7 @@ static int b_rebuild_fwd_table(fl_batch_s* B)
 static void b_free(fl_batch_s* B)
 {
     for (fl_plan pl : B->plans) fl_plan_destroy(pl);
-    void* ptrs[] = {B->d_desc, B->d_fstart, B->d_astart, B->d_vstart, B->r, B->p, B->q, B->sino, B->u, B->part,
+    void* ptrs[] = {B->d_desc, B->d_fstart, B->d_astart, B->d_wstart, B->d_vstart, B->r, B->p, B->q, B->sino, B->u, B->part,
                     B->st, B->log, B->V, B->Dc, B->Atf, B->b};
     for (void* q : ptrs)
         if (q) (void)hipFree(q);
@@ -408,7 +444,7 @@ extern "C" int fl_batch_create(fl_batch* out, int nprob, const fl_geometry* geom
     (void)hipDeviceGetAttribute(&B->cus, hipDeviceAttributeMultiprocessorCount, B->device);
     B->voff.assign(nprob + 1, 0);
     B->soff.assign(nprob + 1, 0);
-    std::vector<int> as(nprob + 1, 0), vs(nprob + 1, 0);
+    std::vector<int> as(nprob + 1, 0), ws(nprob + 1, 0), vs(nprob + 1, 0);
     for (int i = 0; i < nprob; i++) {
         const fl_geometry& g = geoms[i];
         fl_plan pl = nullptr;
@@ -433,19 +469,23 @@ extern "C" int fl_batch_create(fl_batch* out, int nprob, const fl_geometry* geom
         d.n = (int)pl->nvox;
         B->voff[i + 1] = B->voff[i] + pl->nvox;
         B->soff[i + 1] = B->soff[i] + pl->ndet * pl->nv;
-        as[i + 1] = as[i] + ((g.nx + 7) / 8) * ((g.ny + 7) / 8);
+        const int tiles = ((g.nx + 7) / 8) * ((g.ny + 7) / 8);
+        as[i + 1] = as[i] + (d.a.fan_cells ? 0 : tiles);
+        ws[i + 1] = ws[i] + (d.a.fan_cells ? tiles : 0);
         vs[i + 1] = vs[i] + (int)((pl->nvox + CH - 1) / CH);
-        d.adj0 = as[i];
         d.vec0 = vs[i];
         B->desc.push_back(d);
     }
     B->adj_total = as[nprob];
+    B->adjw_total = ws[nprob];
     B->vec_total = vs[nprob];
     hipError_t e = hipMalloc((void**)&B->d_desc, nprob * sizeof(BDesc));
     if (e == hipSuccess) e = hipMalloc((void**)&B->d_fstart, (nprob + 1) * sizeof(int));
     if (e == hipSuccess) e = hipMalloc((void**)&B->d_astart, (nprob + 1) * sizeof(int));
+    if (e == hipSuccess) e = hipMalloc((void**)&B->d_wstart, (nprob + 1) * sizeof(int));
     if (e == hipSuccess) e = hipMalloc((void**)&B->d_vstart, (nprob + 1) * sizeof(int));
     if (e == hipSuccess) e = hipMemcpy(B->d_astart, as.data(), as.size() * sizeof(int), hipMemcpyHostToDevice);
+    if (e == hipSuccess) e = hipMemcpy(B->d_wstart, ws.data(), ws.size() * sizeof(int), hipMemcpyHostToDevice);
     if (e == hipSuccess) e = hipMemcpy(B->d_vstart, vs.data(), vs.size() * sizeof(int), hipMemcpyHostToDevice);
     if (e == hipSuccess) e = hipStreamCreateWithFlags(&B->stream, hipStreamNonBlocking);
     if (e == hipSuccess) e = hipEventCreateWithFlags(&B->ev_in, hipEventDisableTiming);
@@ -462,7 +502,7 @@ extern "C" int fl_batch_create(fl_batch* out, int nprob, const fl_geometry* geom
         return rc;
     }
     B->fwd_grid = 4 * B->cus;
-    B->adj_grid = 4 * B->cus;
+    B->adj_grid = 16 * B->cus;
     B->vec_grid = 2 * B->cus;
     *out = B;
     return fl_ok();
@@ -501,11 +541,20 @@ static int b_forward(fl_batch_s* B, const float* x, float* y, bool gao, hipStrea
 
 static int b_adjoint(fl_batch_s* B, const float* y, float* x, bool matched, hipStream_t st)
 {
-    const unsigned g = (unsigned)std::min(B->adj_grid, std::max(1, B->adj_total));
-    if (matched)
-        hipLaunchKernelGGL(k_badj<true>, dim3(g), dim3(64), 0, st, y, x, B->d_desc, B->d_astart, B->P, B->adj_total);
-    else
-        hipLaunchKernelGGL(k_badj<false>, dim3(g), dim3(64), 0, st, y, x, B->d_desc, B->d_astart, B->P, B->adj_total);
+    if (B->adjw_total) {
+        const dim3 gw((unsigned)std::min(B->adj_grid, B->adjw_total)), bw(64 * (FAN_W + 1));
+        if (matched)
+            hipLaunchKernelGGL(k_badj_w<FanMatched>, gw, bw, 0, st, y, x, B->d_desc, B->d_wstart, B->P, B->adjw_total);
+        else
+            hipLaunchKernelGGL(k_badj_w<FanExact>, gw, bw, 0, st, y, x, B->d_desc, B->d_wstart, B->P, B->adjw_total);
+    }
+    if (B->adj_total) {
+        const dim3 g((unsigned)std::min(B->adj_grid, B->adj_total));
+        if (matched)
+            hipLaunchKernelGGL(k_badj<true>, g, dim3(64), 0, st, y, x, B->d_desc, B->d_astart, B->P, B->adj_total);
+        else
+            hipLaunchKernelGGL(k_badj<false>, g, dim3(64), 0, st, y, x, B->d_desc, B->d_astart, B->P, B->adj_total);
+    }
     BCHK(hipGetLastError());
     return FL_OK;
 }

@@ -75,7 +75,7 @@ static void plan_free_arrays(fl_plan_s* p)
                     p->d_cdet, p->d_sdet, p->d_slot_view, p->d_view_frame, p->d_idY, p->d_idS, p->d_Nv,
                     p->d_bricks,
                     p->d_fb_px, p->d_fb_py, p->d_fb_pd, p->d_cdet2, p->d_sdet2, p->d_line_q,
-                    p->d_ray_q};
+                    p->d_line_d, p->d_fan_views, p->d_ray_q, p->d_ray_l};
     for (void* q : ptrs)
         if (q) (void)hipFree(q);
     if (p->fwd_done) (void)hipEventDestroy(p->fwd_done);
@@ -148,6 +148,63 @@ static int cone_ref_window_bits(const fl_geometry* g, double pa, double pb, cons
         if (!(pb > 0 && g->dz_det > 0 && geo > 1e-3 * SO && fabs(off) + slack < 0.8)) bits |= 2;
     }
     return bits;
+}
+
+// Cells a pixel's shadow can meet on a fan plan's detector, for the windowed
+// adjoints (fl_fan_first_cell); 0 where they must not be used.  The windowed
+// form evaluates every cell of the shadow widened by `margin` cells, which
+// holds every cell of non-zero chord or coefficient, and gives the reference's
+// sum if the reference's window (Atx_fan_mf_cpu_new.cpp:41-47) holds them too.
+// That needs: the shadow inside (|yr| + 1) SD / D (the condition of
+// cone_ref_window_bits), whose index map floors on both sides, so that its
+// constant offset may lie within (-1, 0) less the margins; detector cells
+// on a uniform grid, angle tables that point at them to 0.02 cells, and the
+// adjoint's view angles equal to the forward's (the matched adjoint's) to
+// 0.01 cells; and a margin far above the rounding of a chord's distance test
+// (some 3e-7 (SO + rc)).
+static int fan_shadow_cells(const fl_geometry* g, double pa, double det_dev, const std::vector<float>& cphi,
+                            const std::vector<float>& sphi, const std::vector<float>& cs,
+                            const std::vector<float>& sn, const std::vector<float>& cdet,
+                            const std::vector<float>& sdet, AdjGeom& out)
+{
+    const double margin = 0.05, SO = g->SO, SD = (double)g->SO + g->OD;
+    double ex = 0.0;
+    for (size_t v = 0; v < cphi.size(); v++) {
+        const double c = cphi[v], s = sphi[v];
+        if (!(fabs(c * c + s * s - 1.0) < 1e-5)) return 0;
+        ex = fmax(ex, 0.5 * (fabs(c) + fabs(s)));
+    }
+    const double rc = 0.5 * sqrt((double)(g->nx - 1) * (g->nx - 1) + (double)(g->ny - 1) * (g->ny - 1));
+    const double dmin = SO - rc - 0.01;   // below every pixel centre's depth
+    if (!(pa > 0) || !(g->dy_det > 0) || !(det_dev <= FL_DET_DEV_MAX) || !(dmin > 4 * ex)) return 0;
+    for (size_t v = 0; v < cphi.size(); v++)
+        if (!(fmax(fabs(cphi[v] - cs[v]), fabs(sphi[v] - sn[v])) * 2 * (rc + 1) * SD / dmin < 0.01 * pa)) return 0;
+    for (int a = 0; a < g->na; a++) {
+        const double c = cdet[a], s = sdet[a];
+        if (!(c > 0) || !(fabs(c * c + s * s - 1.0) < 1e-5) || !(fabs(SD * s / c - g->y_det[a]) < 0.02 * pa)) return 0;
+    }
+    const double geo = (1 - ex) * SO - ex - rc * sqrt((1 - ex) * (1 - ex) + ex * ex);
+    const double slack = fabs(1.0 / pa - 1.0 / g->dy_det) * (rc + 1) * SD / dmin + margin + 0.05;
+    const double off = -(double)g->y_det[0] / pa + g->y_os - (double)(g->na / 2);
+    if (!(geo > 1e-3 * SO) || !(off + slack < 0) || !(slack - off < 1)) return 0;
+    if (!((margin - 0.04) * 0.9 * pa * dmin / SD > 1e-6 * (SO + rc))) return 0;
+    const double gr = 1.0 + ex / (dmin - ex);   // 1/(1 + dx/D) of a pixel's corner
+    const double tg = rc / sqrt(SO * SO - rc * rc);
+    const double hmax = sqrt(0.5 * (1.0 + tg * tg)) * gr * (1.0 + 1e-5);
+    const double cells = 2.0 * hmax * SD / dmin / pa + 2 * margin + 1e-3;
+    // the shadow of a tile's pixels: centres within e of the tile's (whose own
+    // may lie that far beyond the image's corner)
+    const double e = 3.5 * 2 * ex, dtile = dmin - 2 * e;
+    if (!(dtile > e) || !(cells < 7)) return 0;
+    const double tile = (2 * e * (1 + tg + e / dtile) + 2 * hmax) * SD / dtile / pa;
+    int n = (int)floor(cells) + 1;
+    n = n <= 2 ? 2 : n <= 4 ? n : n <= 6 ? 6 : 0;   // the instantiated counts
+    out.fan_tile = (int)tile + 4 + n;
+    out.fan_grow = (float)(0.5 * gr * (1.0 + 1e-5));
+    out.fan_hmax = (float)hmax;
+    out.fan_sdp = (float)(SD / pa);
+    out.fan_klo = (float)(-(double)g->y_det[0] / pa - margin);
+    return n <= g->na && out.fan_tile <= 64 ? n : 0;
 }
 
 extern "C" int fl_plan_create(fl_plan* out, const fl_geometry* g)
@@ -367,11 +424,29 @@ extern "C" int fl_plan_create(fl_plan* out, const fl_geometry* g)
         }
     }
     if (!cone) {
-        // the fan adjoint's per-line quotients, built once on the device
-        hipError_t e = hipMalloc((void**)&p->d_line_q, (size_t)g->nv * g->na * sizeof(float2));
+        std::vector<FanView> fv(idY.size(), FanView{1.0f, 0.0f, 1.0f, 0.0f, 0, 0});   // entries past Nv stay unread
+        for (int it = 0; it < g->nt; it++)
+            for (int j = 0; j < Nv[it]; j++) {
+                const size_t k = (size_t)it * tmp + j;
+                const int v = idY[k];
+                fv[k] = FanView{cphi[v], sphi[v], cs[v], sn[v], v, idS[k]};
+            }
+        if ((rc = upload(&p->d_fan_views, fv.data(), fv.size(), "view list"))) {
+            plan_free_arrays(p);
+            delete p;
+            return rc;
+        }
+        a.fan_views = p->d_fan_views;
+        a.fan_cells = fan_shadow_cells(g, g->na > 1 ? ((double)g->y_det[g->na - 1] - g->y_det[0]) / (g->na - 1)
+                                                    : (double)g->dy_det,
+                                       p->det_dev, cphi, sphi, cs, sn, cdet, sdet, a);
+        // the fan adjoint's lines and their quotients, built once on the device
+        hipError_t e = hipMalloc((void**)&p->d_line_q, (size_t)g->nv * g->na * sizeof(float4));
+        if (e == hipSuccess) e = hipMalloc((void**)&p->d_line_d, (size_t)g->na * sizeof(float));
         if (e == hipSuccess) e = hipMalloc((void**)&p->d_ray_q, (size_t)g->nv * g->na * sizeof(float4));
-        if (e == hipSuccess) e = fl_launch_fan_line_q(p->ag, g->nv, p->d_line_q, nullptr);
-        if (e == hipSuccess) e = fl_launch_fan_ray_q(p->fg, g->nv, p->d_ray_q, nullptr);
+        if (e == hipSuccess) e = hipMalloc((void**)&p->d_ray_l, (size_t)g->nv * g->na * sizeof(float));
+        if (e == hipSuccess) e = fl_launch_fan_line_q(p->ag, g->nv, p->d_line_q, p->d_line_d, nullptr);
+        if (e == hipSuccess) e = fl_launch_fan_ray_q(p->fg, g->nv, p->d_ray_q, p->d_ray_l, nullptr);
         if (e == hipSuccess) e = hipStreamSynchronize(nullptr);
         if (e != hipSuccess) {
             plan_free_arrays(p);
@@ -379,7 +454,9 @@ extern "C" int fl_plan_create(fl_plan* out, const fl_geometry* g)
             return fl_hip_fail(e, "fan line quotients");
         }
         a.line_q = p->d_line_q;
+        a.line_d = p->d_line_d;
         a.ray_q = p->d_ray_q;
+        a.ray_l = p->d_ray_l;
     }
     if (cone && !(g->dy_det > 0 && g->dz_det > 0)) {
         plan_free_arrays(p);
@@ -595,7 +672,7 @@ extern "C" int fl_adjoint(fl_plan p, const void* d_y, int yt, void* d_x, int xt,
     hipError_t e;
     if (kind == FL_ADJ_EXACT) {
         e = p->cone ? fl_launch_adj_cone(d_y, yt, d_x, xt, p->ag, st)
-                    : fl_launch_adj_fan(d_y, yt, d_x, xt, p->ag, st);
+                    : fl_launch_adj_fan(d_y, yt, d_x, xt, p->fg, p->ag, st);
     } else if (kind == FL_ADJ_MATCHED) {
         e = fl_launch_adj_matched(d_y, yt, d_x, xt, p, st);
     } else if (kind == FL_ADJ_FAN_FB) {

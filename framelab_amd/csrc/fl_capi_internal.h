@@ -32,8 +32,11 @@ struct fl_plan_s {
     // edge tables (built on first use / uploaded when given)
     float *d_fb_px = nullptr, *d_fb_py = nullptr, *d_fb_pd = nullptr;
     float *d_cdet2 = nullptr, *d_sdet2 = nullptr;
-    float2* d_line_q = nullptr;   // fan: per (view, cell) line-chord quotients
-    float4* d_ray_q = nullptr;    // fan: per (view, cell) ray reciprocals and length
+    float4* d_line_q = nullptr;   // fan: per (view, cell) line and its quotients
+    float* d_line_d = nullptr;    // fan: per cell the lines' right-hand side
+    FanView* d_fan_views = nullptr;
+    float4* d_ray_q = nullptr;    // fan: per (view, cell) ray direction and reciprocals
+    float* d_ray_l = nullptr;     // fan: per (view, cell) ray length
     std::vector<float> h_ydet, h_zdet, h_sdz;
     // largest distance, in cells, of a detector coordinate from the uniform
     // grid through the first and last cell: the adjoints' window maps assume
@@ -66,9 +69,10 @@ hipError_t fl_launch_fwd_fan_gao(const void* X, int xt, void* Y, int yt, const F
 hipError_t fl_launch_trace(const FwdGeom& g, int cone, int nrays, const int* rays, const int* off,
                            const int* cap, int* J, float* S, int* cnt, hipStream_t st);
 hipError_t fl_launch_ynorm(const float* y, float* yn, const FwdGeom& g, hipStream_t st);
-hipError_t fl_launch_adj_fan(const void* Y, int yt, void* X, int xt, const AdjGeom& g, hipStream_t st);
-hipError_t fl_launch_fan_line_q(const AdjGeom& g, int nv, float2* out, hipStream_t st);
-hipError_t fl_launch_fan_ray_q(const FwdGeom& f, int nv, float4* out, hipStream_t st);
+hipError_t fl_launch_adj_fan(const void* Y, int yt, void* X, int xt, const FwdGeom& f, const AdjGeom& g,
+                             hipStream_t st);
+hipError_t fl_launch_fan_line_q(const AdjGeom& g, int nv, float4* out, float* pd, hipStream_t st);
+hipError_t fl_launch_fan_ray_q(const FwdGeom& f, int nv, float4* out, float* len, hipStream_t st);
 hipError_t fl_launch_adj_cone(const void* Y, int yt, void* X, int xt, const AdjGeom& g, hipStream_t st);
 hipError_t fl_launch_adj_matched(const void* Y, int yt, void* X, int xt, const fl_plan_s* p, hipStream_t st);
 hipError_t fl_launch_fwd_fan_fb(const float* X, float* Y, const fl_plan_s* p, hipStream_t st);

@@ -2,8 +2,6 @@
 //
 // Same float arithmetic as the reference chord routines, so the voxel-driven
 // adjoints are bit-identical to the reference's:
-//   fl_chord_line2  <- matlab/mex/src/find_l.cpp:18-45 (line a*x+b*y=c through
-//                      the unit pixel at (x,y));
 //   fl_chord_seg2   <- matlab/mex/src/find_l_3d.cpp:19-92 (segment-line
 //                      through a dx-by-dy cell);
 //   fl_chord_box3   <- matlab/mex/src/find_l_3d.cpp:94-182 (line through a
@@ -21,39 +19,6 @@
 #endif
 
 FL_HD float fl_absf(float v) { return v > 0 ? v : -v; }
-
-FL_HD float fl_chord_line2(float a, float b, float c, float x, float y)
-{
-    float a2 = fl_absf(a), b2 = fl_absf(b);
-    float hx = a2 / 2, hy = b2 / 2;
-    float dmax = hx + hy;
-    float t = c - a * x - b * y;
-    float d = fl_absf(t);
-    float l = 0.0f;
-    if (d < dmax) {
-        float d0 = fl_absf(hx - hy);
-        float flat = (hx < hy) ? 1.0f / b2 : 1.0f / a2;
-        l = (d <= d0) ? flat : (dmax - d) / (a2 * b2);
-    }
-    return l;
-}
-
-// fl_chord_line2 with the line's own quotients supplied, q = (1/max(|a|,
-// |b|), RN(1/(|a||b|))) (the same for every pixel a line meets): the flat
-// value is q.x itself, and (dmax - d)/(|a||b|) is formed from q.y by the
-// Markstein correction, bit-identical to the division.
-__device__ __forceinline__ float fl_chord_line2_q(float a, float b, float c, float x, float y, float2 q)
-{
-    float a2 = fl_absf(a), b2 = fl_absf(b);
-    float hx = a2 / 2, hy = b2 / 2;
-    float dmax = hx + hy;
-    float t = c - a * x - b * y;
-    float d = fl_absf(t);
-    float d0 = fl_absf(hx - hy);
-    const float slope = fl_div_r(dmax - d, a2 * b2, q.y);
-    const float l = (d <= d0) ? q.x : slope;
-    return d < dmax ? l : 0.0f;
-}
 
 FL_HD float fl_chord_seg2(float x1, float y1, float x2, float y2, float dx, float dy, float x, float y)
 {

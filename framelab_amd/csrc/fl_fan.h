@@ -123,12 +123,46 @@ __device__ __forceinline__ float fl_fan_gao_sum(const VT* __restrict__ x, const 
     return acc * g.scale;
 }
 
-// Exact pixel-driven adjoint of pixel (ix, iy) of frame it, scaled
+// Element k of a row, by a 32-bit byte offset from the (wave-uniform) row.
+template <typename T>
+__device__ __forceinline__ const T* fl_row_at(const T* row, unsigned k)
+{
+    return (const T*)((const char*)row + k * (unsigned)sizeof(T));
+}
+
+// ---- pixel-driven adjoints, general form -----------------------------------
+//
+// Per pixel and view a loop over the cells of a window on the detector.  The
+// plans whose geometry bounds a pixel's shadow to a few cells take the
+// windowed form instead (fl_fan_adj.h), which shares the arithmetic of a cell.
+
+// Exact adjoint: the term of one cell, the chord of its line a x + b y = d
+// through the unit pixel at (xc, yc) (find_l.cpp:18-45) times the sinogram
+// value (Atx_fan_mf_cpu_new.cpp:48-58: added only where the chord is
+// positive, which is where the line passes within dmax = (|a| + |b|)/2).
+// ln = (2a, 2b, 1/max(|a|,|b|), 1/(4|a||b|)), pd2 = 2d: the factors of two
+// scale every intermediate exactly (t2 = 2t, num = 4(dmax - |t|), and num
+// and den in the quotient num/den alike) and save the halvings.
+__device__ __forceinline__ float fl_fan_exact_term(float4 ln, float pd2, float xc, float yc, float yv)
+{
+    const float a2 = fabsf(ln.x), b2 = fabsf(ln.y);
+    const float t2 = fabsf(pd2 - ln.x * xc - ln.y * yc);
+    const float num = __builtin_fmaf(-2.0f, t2, a2 + b2);
+    // flat part of the chord: |t| <= ||a| - |b||/2
+    const bool flat = __builtin_fmaf(-2.0f, t2, fabsf(a2 - b2)) >= 0.0f;
+    // (dmax - |t|)/(|a||b|) by Markstein's correction of the tabulated
+    // reciprocal (fl_div_r); where |a||b| is 0 or its reciprocal overflows,
+    // |a| + |b| = ||a| - |b|| in float and the flat value is taken
+    const float den = a2 * b2;
+    const float q = num * ln.w;
+    const float slope = __builtin_fmaf(__builtin_fmaf(-q, den, num), ln.w, q);
+    const float l = flat ? ln.z : slope;
+    return num > 0.0f ? l * yv : 0.0f;
+}
+
+// General exact adjoint of pixel (ix, iy) of frame it, scaled
 // (Atx_fan_mf_cpu_new.cpp:35-62).
-// LQ: take the lines' pixel-independent quotients from g.line_q (one table
-// read per cell instead of up to three divisions); the batched kernel,
-// whose small persistent workgroups hide the extra read worse, divides.
-template <typename YT, bool LQ = true>
+template <typename YT>
 __device__ __forceinline__ float fl_fan_adj_pixel(const YT* __restrict__ Y, const AdjGeom& g, int it, int ix, int iy)
 {
     const int nd = g.na, nd2 = nd / 2;
@@ -148,18 +182,9 @@ __device__ __forceinline__ float fl_fan_adj_pixel(const YT* __restrict__ Y, cons
         int lo = (int)floorf((yr - 1) * t - g.y_os + (float)nd2);
         if (lo < 0) lo = 0;
         if (hi > nd - 1) hi = nd - 1;
-        const float2* __restrict__ lq = LQ ? g.line_q + (size_t)iv * nd : nullptr;
-        for (int id = lo; id <= hi; id++) {
-            const float sd = g.sdet[id], cd = g.cdet[id];
-            const float Px = -(sd * c + cd * s);
-            const float Py = cd * c - sd * s;
-            const float Pd = g.SO * sd;
-            const float l = LQ ? fl_chord_line2_q(Px, Py, Pd, xc, yc, lq[id]) : fl_chord_line2(Px, Py, Pd, xc, yc);
-            // a select, not a branch around the load: lanes of a wave
-            // disagree on l > 0 too often for a branch to pay
-            const float yv = fl_load(y, (size_t)id);
-            acc = l > 0 ? acc + l * yv : acc;
-        }
+        const float4* __restrict__ line = g.line_q + (size_t)iv * nd;
+        for (int id = lo; id <= hi; id++)
+            acc = acc + fl_fan_exact_term(line[id], g.line_d[id], xc, yc, fl_load(y, (size_t)id));
     }
     return acc * g.scale;
 }
@@ -202,10 +227,35 @@ __device__ __forceinline__ FlAxisIv fl_slab_r(const SidAxis& a, int cell, float 
     return r;
 }
 
-// Matched (Siddon-transpose) adjoint of pixel (ix, iy) of frame it, scaled.
-// RQ: take each ray's reciprocals and length from g.ray_q instead of
-// forming them per pixel (same values, the same IEEE operations made once).
-template <typename YT, bool RQ = true>
+// Matched adjoint: the term of one cell for a pixel whose x planes lie at xl,
+// xl + 1 and y planes at yl, yl + 1 from the source (x1, y1): the Siddon
+// segment of the ray inside the pixel, credited where the forward's midpoint
+// rule maps it there, times the sinogram value.  r4 = (dx, dy, 1/dx, 1/dy) of
+// the ray, 0 in place of the reciprocal of a zero component (the ray is
+// parallel to that axis' planes), L its length.  Plane parameters are the
+// forward's quotients (fl_div_r); every test is evaluated, without branches.
+__device__ __forceinline__ float fl_fan_matched_term(float4 r4, float L, float xl, float xh, float yl, float yh,
+                                                     float x1, float y1, float nhx, float nhy, int ix, int iy, float yv)
+{
+    auto quot = [](float num, float d, float r) {
+        const float q = num * r;
+        return __builtin_fmaf(__builtin_fmaf(-q, d, num), r, q);
+    };
+    const float ax = quot(xl, r4.x, r4.z), bx = quot(xh, r4.x, r4.z);
+    const float ay = quot(yl, r4.y, r4.w), by = quot(yh, r4.y, r4.w);
+    const bool onx = r4.x != 0.0f, ony = r4.y != 0.0f;
+    const float inx = onx ? fminf(ax, bx) : -FL_INF, outx = onx ? fmaxf(ax, bx) : FL_INF;
+    const float iny = ony ? fminf(ay, by) : -FL_INF, outy = ony ? fmaxf(ay, by) : FL_INF;
+    const float ain = fmaxf(inx, iny), aout = fminf(outx, outy);
+    const float m = (ain + aout) * 0.5f;
+    const int tx = (int)floorf(x1 + m * r4.x + nhx), ty = (int)floorf(y1 + m * r4.y + nhy);
+    const int hit = int(aout > ain) & int(tx == ix) & int(ty == iy);
+    return hit ? ((aout - ain) * L) * yv : 0.0f;
+}
+
+// General matched (Siddon-transpose) adjoint of pixel (ix, iy) of frame it,
+// scaled.
+template <typename YT>
 __device__ __forceinline__ float fl_fan_matched_pixel(const YT* __restrict__ Y, const FwdGeom& f, const AdjGeom& g,
                                                       int it, int ix, int iy)
 {
@@ -213,6 +263,7 @@ __device__ __forceinline__ float fl_fan_matched_pixel(const YT* __restrict__ Y, 
     const float SD = f.SO + f.OD;
     const float xc = (float)ix + 0.5f - (float)(f.nx / 2);
     const float yc = (float)iy + 0.5f - (float)(f.ny / 2);
+    const float nhx = (float)(f.nx / 2), nhy = (float)(f.ny / 2);
     const float ya0 = f.ydet[0];
     float acc = 0.0f;
     const int nvf = g.Nv[it];
@@ -228,24 +279,13 @@ __device__ __forceinline__ float fl_fan_matched_pixel(const YT* __restrict__ Y, 
         if (lo < 0) lo = 0;
         if (hi > nd - 1) hi = nd - 1;
         const float x1 = c * (-f.SO), y1 = s * (-f.SO);
-        const float4* __restrict__ rq = RQ ? g.ray_q + (size_t)iv * nd : nullptr;
-        for (int id = lo; id <= hi; id++) {
-            const float yd = f.ydet[id];
-            const float x2 = c * f.OD - s * yd;
-            const float y2 = s * f.OD + c * yd;
-            const float dx = x2 - x1, dy = y2 - y1;
-            const float4 q = RQ ? rq[id] : make_float4(1.0f / dx, 1.0f / dy, 0.0f, 0.0f);
-            SidAxis ax, ay;
-            sid_axis_init(ax, x1, dx, 1.0f, f.nx);
-            sid_axis_init(ay, y1, dy, 1.0f, f.ny);
-            const FlAxisIv sx = fl_slab_r(ax, ix, q.x), sy = fl_slab_r(ay, iy, q.y);
-            const float ain = fmaxf(sx.in, sy.in), aout = fminf(sx.out, sy.out);
-            if (!(aout > ain)) continue;
-            const float m = (ain + aout) * 0.5f;
-            if (sid_cell_xy(ax, m) != ix || sid_cell_xy(ay, m) != iy) continue;
-            const float L = RQ ? q.z : sqrtf(dx * dx + dy * dy);
-            acc = acc + ((aout - ain) * L) * fl_load(y, (size_t)id);
-        }
+        const float xl = (float)(ix - f.nx / 2) - x1, xh = (float)(ix - f.nx / 2 + 1) - x1;
+        const float yl = (float)(iy - f.ny / 2) - y1, yh = (float)(iy - f.ny / 2 + 1) - y1;
+        const float4* __restrict__ ray = g.ray_q + (size_t)iv * nd;
+        const float* __restrict__ len = g.ray_l + (size_t)iv * nd;
+        for (int id = lo; id <= hi; id++)
+            acc = acc + fl_fan_matched_term(ray[id], len[id], xl, xh, yl, yh, x1, y1, nhx, nhy, ix, iy,
+                                            fl_load(y, (size_t)id));
     }
     return acc * f.scale;
 }

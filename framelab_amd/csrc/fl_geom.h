@@ -21,6 +21,14 @@ struct FwdGeom {
     void* bricks;           // cone: bricked copy of the input frames (plan-owned)
 };
 
+// One entry of a fan plan's frame -> views lists: what the pixel-driven
+// adjoints need of the view, in one scalar read.
+struct alignas(32) FanView {
+    float c, s;        // para.cos_phi, para.sin_phi
+    float cf, sf;      // the forward's cosf(sd_phi), sinf(sd_phi)
+    int view, slot;    // view index, sinogram slot the forward writes it to
+};
+
 // Voxel-driven adjoint geometry (the reference para tables).
 struct AdjGeom {
     const float* cphi;      // para.cos_phi
@@ -43,9 +51,22 @@ struct AdjGeom {
     // reference's detector window may cut a voxel's shadow window and has
     // to be applied; clear where the plan's geometry rules that out
     int win_ref;
-    // fan: per (view, cell) the view-only quotients of the line chord,
-    // (1/max(|a|,|b|), 1/(|a||b|)), at [iv*nd + id]
-    const float2* line_q;
-    // fan: per (view, cell) (1/dx, 1/dy, |d|) of the ray, for the matched adjoint
+    // fan: per (view, cell) the line a x + b y = d and its pixel-independent
+    // quotients, (2a, 2b, 1/max(|a|,|b|), 1/(4|a||b|)), at [iv*nd + id]; 2d per
+    // cell (fl_fan_exact_term)
+    const float4* line_q;
+    const float* line_d;
+    // fan: frame -> views (id_Y's layout)
+    const FanView* fan_views;
+    // fan, windowed adjoints (fl_fan_adj.h): cells a pixel's shadow can meet,
+    // 0 where the plan's geometry gives no small bound; cells the shadow of an
+    // 8 x 8 tile can; the shadow's perspective factor (times 1/2) and largest
+    // half width; SD over the pitch and the index map's offset of a shadow's
+    // lower edge
+    int fan_cells, fan_tile;
+    float fan_grow, fan_hmax, fan_sdp, fan_klo;
+    // fan: per (view, cell) (dx, dy, 1/dx, 1/dy) of the ray (0 for the
+    // reciprocal of a zero component) and its length, for the matched adjoint
     const float4* ray_q;
+    const float* ray_l;
 };

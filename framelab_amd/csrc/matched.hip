@@ -23,6 +23,7 @@
 #include "fl_siddon.h"
 #include "fl_chord.h"
 #include "fl_fan.h"
+#include "fl_fan_adj.h"
 
 // Workgroups per CU the register budget is sized for (a build-time tuning
 // knob; the default is the measured optimum at 256^3).
@@ -277,6 +278,7 @@ __global__ __launch_bounds__(256, FL_MATCHED_WG_PER_CU) void k_adj_matched_cone(
     }
 }
 
+// General form: one lane per pixel.
 template <typename YT, typename XT>
 __global__ __launch_bounds__(256) void k_adj_matched_fan(const YT* __restrict__ Y, XT* __restrict__ X,
                                                         FwdGeom f, AdjGeom g)
@@ -303,8 +305,9 @@ static hipError_t launch_matched_t(const void* Y, void* X, const fl_plan_s* p, h
                                (const YT*)Y, (XT*)X, f, p->ag);
     } else {
         dim3 grid((f.nx + 15) / 16, (f.ny + 15) / 16, p->nt);
-        hipLaunchKernelGGL((k_adj_matched_fan<YT, XT>), grid, dim3(16, 16), 0, st, (const YT*)Y, (XT*)X, f,
-                           p->ag);
+        if (!fl_launch_fan_adj_w<FanMatched>((const YT*)Y, (XT*)X, f, p->ag, st))
+            hipLaunchKernelGGL((k_adj_matched_fan<YT, XT>), grid, dim3(16, 16), 0, st, (const YT*)Y, (XT*)X, f,
+                               p->ag);
     }
     return hipGetLastError();
 }
