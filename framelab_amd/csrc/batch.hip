@@ -55,6 +55,10 @@ __device__ __forceinline__ int find_problem(const int* __restrict__ start, int P
 
 // ---------------------------------------------------------------- operators
 
+// An item is T rays: T/FV cells of FV neighbouring views, walked by waves of
+// FAN_WA cells x FV views (fl_fan.h).
+constexpr int FV = 64 / FAN_WA;
+
 template <bool GAO>
 __global__ __launch_bounds__(64) void k_bfwd(const float* __restrict__ X, float* __restrict__ Y,
                                             const BDesc* __restrict__ D, const int* __restrict__ start, int P,
@@ -63,18 +67,24 @@ __global__ __launch_bounds__(64) void k_bfwd(const float* __restrict__ X, float*
     for (int item = blockIdx.x; item < total; item += gridDim.x) {
         const int p = find_problem(start, P, item);
         const FwdGeom f = D[p].f;
-        const long long voff = D[p].voff, soff = D[p].soff;
         const int local = item - start[p];
-        const int tpv = (f.na + T - 1) / T;
-        const int slot = local / tpv, t = local % tpv;
-        const int iv = f.slot_view[slot];
-        const float* x = X + voff + (size_t)f.view_frame[iv] * f.nvox;
-        for (int k = threadIdx.x; k < T; k += 64) {
-            const int id = t * T + k;
-            if (id < f.na) {
-                const float v = GAO ? fl_fan_gao_sum(x, f, iv, id) : fl_fan_ray_sum(x, f, iv, id);
-                Y[soff + (size_t)slot * f.na + id] = v;
+        const int tc = T / FV, tpv = (f.na + tc - 1) / tc;
+        const int slot = local / tpv * FV + (int)threadIdx.x / FAN_WA, t = local % tpv;
+        const int iv = f.slot_view[min(slot, f.nslots - 1)];
+        const float* x = X + D[p].voff + (size_t)f.view_frame[iv] * f.nvox;
+        float* y = Y + D[p].soff + (size_t)slot * f.na;
+        for (int k = 0; k < tc; k += FAN_WA) {
+            const int id = t * tc + k + (int)threadIdx.x % FAN_WA;
+            const bool live = slot < f.nslots && id < f.na;
+            float v = 0.0f;
+            if (GAO) {
+                if (live) v = fl_fan_gao_sum(x, f, iv, id);
+            } else if (fl_fan_small(f.nx, f.ny)) {
+                v = fl_fan_ray_sum<true>(x, f, iv, min(id, f.na - 1), live);
+            } else {
+                v = fl_fan_ray_sum<false>(x, f, iv, min(id, f.na - 1), live);
             }
+            if (live) y[id] = v;
         }
     }
 }
@@ -400,7 +410,8 @@ static int b_rebuild_fwd_table(fl_batch_s* B)
     std::vector<int> fs(B->P + 1, 0);
     for (int i = 0; i < B->P; i++) {
         const FwdGeom& f = B->desc[i].f;
-        fs[i + 1] = fs[i] + f.nslots * ((f.na + B->T - 1) / B->T);
+        const int tc = B->T / FV;
+        fs[i + 1] = fs[i] + (f.nslots + FV - 1) / FV * ((f.na + tc - 1) / tc);
         B->desc[i].fwd0 = fs[i];
     }
     B->fwd_total = fs[B->P];
@@ -501,7 +512,7 @@ extern "C" int fl_batch_create(fl_batch* out, int nprob, const fl_geometry* geom
         delete B;
         return rc;
     }
-    B->fwd_grid = 4 * B->cus;
+    B->fwd_grid = 32 * B->cus;
     B->adj_grid = 16 * B->cus;
     B->vec_grid = 2 * B->cus;
     *out = B;

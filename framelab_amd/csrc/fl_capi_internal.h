@@ -54,6 +54,7 @@ struct fl_plan_s {
 constexpr int FL_FWD_NTILES = 8;   // cone forward ray-tile shapes (siddon.hip)
 // elements of the largest bricked frame of any of them (siddon.hip)
 size_t fl_bricked_frame_elems(int nx, int ny, int nz);
+size_t fl_tracked_frame_elems(int nx, int ny, int nz);
 // detector coordinates may stray from a uniform grid by at most this many
 // cells for the voxel-driven adjoints (their windows widen by 0.05 cells)
 constexpr double FL_DET_DEV_MAX = 0.01;

@@ -76,6 +76,18 @@ __device__ __forceinline__ void fl_store_nt(f16_t* p, size_t i, float v)
     __builtin_nontemporal_store((_Float16)v, &p[i].v);
 }
 
+// A stored value held until it is used: 32 bits wide, so that reads in flight
+// need no merging of register halves.
+__device__ __forceinline__ float fl_raw(const float* p) { return *p; }
+__device__ __forceinline__ uint32_t fl_raw(const bf16_t* p) { return p->v; }
+__device__ __forceinline__ uint32_t fl_raw(const f16_t* p) { return *(const uint16_t*)p; }
+__device__ __forceinline__ float fl_unraw(const float*, float v) { return v; }
+__device__ __forceinline__ float fl_unraw(const bf16_t*, uint32_t v) { return __uint_as_float(v << 16); }
+__device__ __forceinline__ float fl_unraw(const f16_t*, uint32_t v)
+{
+    return (float)__builtin_bit_cast(_Float16, (uint16_t)v);
+}
+
 // Map a linear workgroup id so that consecutive logical tiles land on the
 // same XCD (the dispatcher deals workgroups round-robin over 8 XCDs, each
 // with its own L2).  nblk must be the grid size along the remapped axis.

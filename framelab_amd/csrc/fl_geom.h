@@ -19,6 +19,7 @@ struct FwdGeom {
     float ya0, inv_pa, zb0, inv_pb;
     int tile;               // cone forward launch shape, 0..FL_FWD_NTILES-1
     void* bricks;           // cone: bricked copy of the input frames (plan-owned)
+    bool tracked;           // cone: it has room for the tracked walk's padded layout
 };
 
 // One entry of a fan plan's frame -> views lists: what the pixel-driven

@@ -153,20 +153,24 @@ FL_HD void sid_next_step(SidNext& n, const SidAxis& ax, float an)
     n.p = adv ? pn : n.p;
 }
 
-// Generic walk over one ray.  NZ3 = true for the cone (3 axes); DZ1 = the
-// z plane spacing is 1 (cell index needs no division).  The visitor
-// receives (linear voxel index (z*ny+y)*nx+x, alpha difference of the
-// segment) for every in-volume segment in traversal order; the length is
-// that difference times |d|.
-template <bool NZ3, bool DZ1, bool XYZ, bool ALL = false, class Visit>
-FL_HD void sid_walk_t(const SidAxis& ax, const SidAxis& ay, const SidAxis& az, float L, Visit&& visit)
+// A ray's position in its walk.
+struct SidWalk {
+    SidNext x, y, z;   // next plane per axis
+    float cur;         // parameter of the last plane passed
+};
+
+// The walk's start: false if nothing of the ray is inside the volume.
+// NZ3 = true for the cone (3 axes); DZ1 = the z plane spacing is 1.
+template <bool NZ3, bool DZ1>
+FL_HD bool sid_start(const SidAxis& ax, const SidAxis& ay, const SidAxis& az, SidWalk& w)
 {
     constexpr bool dz_one = DZ1;
     // Inactive axes keep a constant cell index; if it is outside, nothing
     // of the ray is inside the volume.
-    if (!ax.on && !sid_in(ax, sid_cell_xy(ax, 0.5f))) return;
-    if (!ay.on && !sid_in(ay, sid_cell_xy(ay, 0.5f))) return;
-    if (NZ3 && !az.on && !sid_in(az, sid_cell_z(az, 0.5f, dz_one))) return;
+    if (!ax.on && !sid_in(ax, sid_cell_xy(ax, 0.5f))) return false;
+    if (!ay.on && !sid_in(ay, sid_cell_xy(ay, 0.5f))) return false;
+    if (NZ3 && !az.on && !sid_in(az, sid_cell_z(az, 0.5f, dz_one))) return false;
+    if (!ax.on && !ay.on && (!NZ3 || !az.on)) return false;
 
     // Entry parameter: the largest first-plane parameter of the active axes.
     float ae = -FL_INF;
@@ -190,13 +194,36 @@ FL_HD void sid_walk_t(const SidAxis& ax, const SidAxis& ay, const SidAxis& az, f
         if (near) break;
         cur = pred;
     }
+    w.cur = cur;
+    sid_next_init(w.x, ax, ax.on ? sid_count(ax, cur, false) : 0);
+    sid_next_init(w.y, ay, ay.on ? sid_count(ay, cur, false) : 0);
+    if (NZ3) sid_next_init(w.z, az, az.on ? sid_count(az, cur, false) : 0);
+    else w.z.a = FL_INF;
+    return true;
+}
 
-    // Forward walk from `cur`.
-    SidNext qx, qy, qz;
-    sid_next_init(qx, ax, ax.on ? sid_count(ax, cur, false) : 0);
-    sid_next_init(qy, ay, ay.on ? sid_count(ay, cur, false) : 0);
-    if (NZ3) sid_next_init(qz, az, az.on ? sid_count(az, cur, false) : 0);
-    else qz.a = FL_INF;
+// floor to int in one instruction (the walks' midpoints are never NaN).
+FL_HD int sid_floor(float v)
+{
+#if defined(__HIP_DEVICE_COMPILE__)
+    int r;
+    asm("v_cvt_flr_i32_f32 %0, %1" : "=v"(r) : "v"(v));
+    return r;
+#else
+    return (int)floorf(v);
+#endif
+}
+
+// Generic walk over one ray.  The visitor receives (linear voxel index
+// (z*ny+y)*nx+x, alpha difference of the segment) for every in-volume segment
+// in traversal order; the length is that difference times |d|.
+template <bool NZ3, bool DZ1, bool ALL = false, class Visit>
+FL_HD void sid_walk_t(const SidAxis& ax, const SidAxis& ay, const SidAxis& az, float L, Visit&& visit)
+{
+    SidWalk w;
+    if (!sid_start<NZ3, DZ1>(ax, ay, az, w)) return;
+    SidNext &qx = w.x, &qy = w.y, &qz = w.z;
+    float cur = w.cur;
     const float rs = NZ3 && !DZ1 ? 1.0f / az.s : 1.0f;
 
     const int nx = ax.n, ny = ay.n;
@@ -229,8 +256,7 @@ FL_HD void sid_walk_t(const SidAxis& ax, const SidAxis& ay, const SidAxis& az, f
             if (stop) break;
             continue;
         } else if (in) {
-            if constexpr (XYZ) visit(tx, ty, tz, an - cur);
-            else visit((tz * ny + ty) * nx + tx, an - cur);
+            visit((tz * ny + ty) * nx + tx, an - cur);
         } else {
             bool far = sid_far(ax, tx) || sid_far(ay, ty) || (NZ3 && sid_far(az, tz));
             if (far) break;
@@ -245,8 +271,8 @@ FL_HD void sid_walk_t(const SidAxis& ax, const SidAxis& ay, const SidAxis& az, f
 template <bool NZ3, class Visit>
 FL_HD void sid_walk(const SidAxis& ax, const SidAxis& ay, const SidAxis& az, float L, bool dz_one, Visit&& visit)
 {
-    if (dz_one) sid_walk_t<NZ3, true, false>(ax, ay, az, L, visit);
-    else sid_walk_t<NZ3, false, false>(ax, ay, az, L, visit);
+    if (dz_one) sid_walk_t<NZ3, true>(ax, ay, az, L, visit);
+    else sid_walk_t<NZ3, false>(ax, ay, az, L, visit);
 }
 
 // Every step of the walk: tok = visit(tx, ty, tz, dal, in) for the
@@ -257,23 +283,6 @@ template <class Visit>
 FL_HD void sid_walk_all3(const SidAxis& ax, const SidAxis& ay, const SidAxis& az, float L, bool dz_one,
                          Visit&& visit)
 {
-    if (dz_one) sid_walk_t<true, true, true, true>(ax, ay, az, L, visit);
-    else sid_walk_t<true, false, true, true>(ax, ay, az, L, visit);
-}
-
-// The same for a 2-D walk (tz = 0).
-template <class Visit>
-FL_HD void sid_walk_all2(const SidAxis& ax, const SidAxis& ay, const SidAxis& az, float L, Visit&& visit)
-{
-    sid_walk_t<false, true, true, true>(ax, ay, az, L, visit);
-}
-
-// As sid_walk, but the visitor receives the cell coordinates (tx, ty, tz)
-// instead of the linear index.
-template <bool NZ3, class Visit>
-FL_HD void sid_walk_xyz(const SidAxis& ax, const SidAxis& ay, const SidAxis& az, float L, bool dz_one,
-                        Visit&& visit)
-{
-    if (dz_one) sid_walk_t<NZ3, true, true>(ax, ay, az, L, visit);
-    else sid_walk_t<NZ3, false, true>(ax, ay, az, L, visit);
+    if (dz_one) sid_walk_t<true, true, true>(ax, ay, az, L, visit);
+    else sid_walk_t<true, false, true>(ax, ay, az, L, visit);
 }

@@ -14,6 +14,7 @@
 #include "fl_common.h"
 #include "fl_geom.h"
 #include "fl_siddon.h"
+#include "fl_walk.h"
 #include "fl_chord.h"
 #include "fl_fan.h"
 
@@ -98,11 +99,19 @@ struct Bricks {
     }
 };
 
-// Elements of the largest bricked frame of any launch shape (plan buffers).
+// Elements of the largest unpadded bricked frame of any launch shape.
 size_t fl_bricked_frame_elems(int nx, int ny, int nz)
 {
-    return std::max(Bricks<8, 8>(nx, ny, nz).frame,
-                    std::max(Bricks<4, 4, 4>(nx, ny, nz).frame, Bricks<4, 4, 2>(nx, ny, nz).frame));
+    return std::max({Bricks<8, 8>(nx, ny, nz).frame, Bricks<4, 4, 4>(nx, ny, nz).frame, Bricks<4, 4, 2>(nx, ny, nz).frame});
+}
+
+// Elements of the tracked walk's padded frame; 0 where its 32-bit byte offsets
+// do not reach (2^30 voxels and more): such volumes take the unpadded bricks.
+size_t fl_tracked_frame_elems(int nx, int ny, int nz)
+{
+    if (nx >= (1 << 24) || ny >= (1 << 24) || nz >= (1 << 24)) return 0;
+    const size_t frame = ConeBricks<4>(nx, ny).frame(nz);
+    return frame <= ((size_t)1 << 30) ? frame : 0;
 }
 
 // The bricked layouts' index arithmetic needs a brick slab of under 2^24
@@ -186,16 +195,59 @@ __global__ __launch_bounds__(TA* TB) void k_fwd_cone(const VT* __restrict__ X, Y
     fl_store(Y, ((size_t)slot * g.nb + ib) * g.na + ia, acc * g.scale);
 }
 
-template <typename VT, typename YT>
-__global__ __launch_bounds__(64) void k_fwd_fan(const VT* __restrict__ X, YT* __restrict__ Y, FwdGeom g)
+template <typename VT>
+__global__ __launch_bounds__(256) void k_to_cone_bricks(const VT* __restrict__ x, VT* __restrict__ xb, int nx, int ny,
+                                                       int nz, size_t nvox, size_t n)
 {
-    const uint32_t tiles = (g.na + 63) / 64;
+    const ConeBricks<sizeof(VT)> br(nx, ny);
+    const size_t frame = br.frame(nz);
+    for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (size_t)gridDim.x * 256) {
+        const size_t f = i / nvox, v = i % nvox;
+        const int tx = (int)(v % nx), ty = (int)((v / nx) % ny), tz = (int)(v / ((size_t)nx * ny));
+        *(VT*)((char*)(xb + f * frame) + br.at(tx, ty, tz)) = x[i];
+    }
+}
+
+// Cone forward with tracked cells (fl_walk.h): workgroups of 16 x 16 detector
+// cells of one view, waves of 8 x 8.  256^3, 360 views x 512 x 384: 14.05 ms
+// with the cell's indices formed at every step (k_fwd_cone), 8.93 ms so (BF16
+// 14.1 -> 8.0; 128^3, 180 views x 256 x 192: 1.20 -> 0.64 ms): bound by VALU
+// issue, some 29 instructions a step of which 27 cross planes.  Six waves per
+// SIMD: the 80 registers this leaves hold the walk without spills.
+template <typename VT, typename YT, bool DZ1>
+__global__ __launch_bounds__(256, 6) void k_fwd_cone_tr(const VT* __restrict__ X, YT* __restrict__ Y, FwdGeom g)
+{
+    const uint32_t tiles_a = (g.na + 15) / 16, tiles_b = (g.nb + 15) / 16, tpv = tiles_a * tiles_b;
     const uint32_t b = fl_xcd_remap(blockIdx.x, gridDim.x);
-    const int slot = (int)(b / tiles);
-    const int id = (int)(b % tiles) * 64 + (int)threadIdx.x;
-    if (slot >= g.nslots || id >= g.na) return;
+    const int slot = (int)(b / tpv);
+    const uint32_t t = b % tpv;
+    const int w = (int)threadIdx.x >> 6, l = (int)threadIdx.x & 63;
+    const int ia = (int)(t % tiles_a) * 16 + (w & 1) * 8 + l % 8;
+    const int ib = (int)(t / tiles_a) * 16 + (w >> 1) * 8 + l / 8;
+    const bool live = ia < g.na && ib < g.nb;
     const int iv = g.slot_view[slot];
-    fl_store(Y, (size_t)slot * g.na + id, fl_fan_ray_sum(X + (size_t)g.view_frame[iv] * g.nvox, g, iv, id));
+    const ConeBricks<sizeof(VT)> br(g.nx, g.ny);
+    const RayGeo r = cone_ray(g, iv, min(ia, g.na - 1), min(ib, g.nb - 1));
+    WalkAxis ax, ay, az;
+    walk_axis_init(ax, r.x1, r.dx, 1.0f, g.nx);
+    walk_axis_init(ay, r.y1, r.dy, 1.0f, g.ny);
+    walk_axis_init(az, r.z1, r.dz, g.dz0, g.nz);
+    const float acc = walk_rays<true, DZ1, true>(ax, ay, az, r.L, live, X + (size_t)g.view_frame[iv] * br.frame(g.nz), br);
+    if (live) fl_store(Y, ((size_t)slot * g.nb + ib) * g.na + ia, acc * g.scale);
+}
+
+template <typename VT, typename YT, bool SMALL>
+__global__ __launch_bounds__(256) void k_fwd_fan(const VT* __restrict__ X, YT* __restrict__ Y, FwdGeom g)
+{
+    constexpr int WA = FAN_WA, WV = 64 / WA;   // a wave's cells and views
+    const uint32_t tiles = (g.na + 4 * WA - 1) / (4 * WA);
+    const uint32_t b = fl_xcd_remap(blockIdx.x, gridDim.x);
+    const int slot = (int)(b / tiles) * WV + (int)(threadIdx.x & 63) / WA;
+    const int id = (int)(b % tiles) * 4 * WA + (int)(threadIdx.x >> 6) * WA + (int)threadIdx.x % WA;
+    const bool live = slot < g.nslots && id < g.na;
+    const int iv = g.slot_view[min(slot, g.nslots - 1)];
+    const float v = fl_fan_ray_sum<SMALL>(X + (size_t)g.view_frame[iv] * g.nvox, g, iv, min(id, g.na - 1), live);
+    if (live) fl_store(Y, (size_t)slot * g.na + id, v);
 }
 
 // Traversal log of selected rays (parity tests): ray k = (view, ia, ib)
@@ -251,8 +303,25 @@ static hipError_t launch_cone_shape(const void* X, void* Y, const FwdGeom& g, hi
     return hipGetLastError();
 }
 
+template <typename VT, typename YT>
+static hipError_t launch_cone_tr(const void* X, void* Y, const FwdGeom& g, hipStream_t st)
+{
+    const uint32_t grid = (uint32_t)((g.na + 15) / 16) * (uint32_t)((g.nb + 15) / 16) * (uint32_t)g.nslots;
+    if (grid == 0) return hipSuccess;
+    if (!g.tracked) return launch_cone_shape<VT, YT, 16, 16, 8, 4, 4, 4>(X, Y, g, st);
+    const size_t n = g.nvox * (size_t)g.nframes;
+    hipLaunchKernelGGL((k_to_cone_bricks<VT>), dim3((unsigned)std::min<size_t>((n + 255) / 256, 8192)), dim3(256), 0, st,
+                       (const VT*)X, (VT*)g.bricks, g.nx, g.ny, g.nz, g.nvox, n);
+    if (g.dz0 == 1.0f)
+        hipLaunchKernelGGL((k_fwd_cone_tr<VT, YT, true>), dim3(grid), dim3(256), 0, st, (const VT*)g.bricks, (YT*)Y, g);
+    else
+        hipLaunchKernelGGL((k_fwd_cone_tr<VT, YT, false>), dim3(grid), dim3(256), 0, st, (const VT*)g.bricks, (YT*)Y, g);
+    return hipGetLastError();
+}
+
 // Launch shapes, indexed by FwdGeom::tile (fl_plan_autotune times them):
-// workgroup TA x TB rays, waves WA x 64/WA, volume bricks BX x BY x BZ.
+// workgroup TA x TB rays, waves WA x 64/WA, volume bricks BX x BY x BZ; shape
+// 6, the default, walks with tracked cells.
 template <typename VT, typename YT>
 static hipError_t launch_cone_t(const void* X, void* Y, const FwdGeom& g, hipStream_t st)
 {
@@ -269,7 +338,7 @@ static hipError_t launch_cone_t(const void* X, void* Y, const FwdGeom& g, hipStr
     case 3: return launch_cone_shape<VT, YT, 16, 16, 8, 1, 1>(X, Y, g, st);
     case 4: return launch_cone_shape<VT, YT, 16, 16, 8, 4, 4>(X, Y, g, st);
     case 5: return launch_cone_shape<VT, YT, 64, 4, 64, 8, 8>(X, Y, g, st);
-    case 6: return launch_cone_shape<VT, YT, 16, 16, 8, 4, 4, 4>(X, Y, g, st);
+    case 6: return launch_cone_tr<VT, YT>(X, Y, g, st);
     default: return launch_cone_shape<VT, YT, 16, 16, 8, 4, 4, 2>(X, Y, g, st);
     }
 }
@@ -277,9 +346,13 @@ static hipError_t launch_cone_t(const void* X, void* Y, const FwdGeom& g, hipStr
 template <typename VT, typename YT>
 static hipError_t launch_fan_t(const void* X, void* Y, const FwdGeom& g, hipStream_t st)
 {
-    uint32_t grid = ((g.na + 63) / 64) * (uint32_t)g.nslots;
+    const uint32_t grid = (uint32_t)((g.na + 4 * FAN_WA - 1) / (4 * FAN_WA)) *
+                          (uint32_t)((g.nslots + 64 / FAN_WA - 1) / (64 / FAN_WA));
     if (grid == 0) return hipSuccess;
-    hipLaunchKernelGGL((k_fwd_fan<VT, YT>), dim3(grid), dim3(64), 0, st, (const VT*)X, (YT*)Y, g);
+    if (fl_fan_small(g.nx, g.ny))
+        hipLaunchKernelGGL((k_fwd_fan<VT, YT, true>), dim3(grid), dim3(256), 0, st, (const VT*)X, (YT*)Y, g);
+    else
+        hipLaunchKernelGGL((k_fwd_fan<VT, YT, false>), dim3(grid), dim3(256), 0, st, (const VT*)X, (YT*)Y, g);
     return hipGetLastError();
 }
 
