@@ -25,249 +25,411 @@
 #include "fl_fan.h"
 #include "fl_fan_adj.h"
 
-// Workgroups per CU the register budget is sized for (a build-time tuning
-// knob; the default is the measured optimum at 256^3).
-#ifndef FL_MATCHED_WG_PER_CU
-#define FL_MATCHED_WG_PER_CU 5
-#endif
-
-
-
-// Per (ray, voxel) pair of one view: the Siddon segment of the ray inside
-// the voxel, credited when the forward's midpoint rule maps it there.
-// in/out: entry/exit plane parameters per axis.  Returns the length
-// coefficient (a_out - a_in)*|d|, or 0.  Branch-free: the three cell tests
-// cost less than the divergent branches around them.
-__device__ __forceinline__ float matched_coef(float inx, float outx, float iny, float outy, float inz, float outz,
-                                              const SidAxis& ax, const SidAxis& ay, const SidAxis& az, int ix,
-                                              int iy, int iz, bool dz_one, float L)
+// Per (ray, voxel) pair: the length (in parameter) of the Siddon segment of the
+// ray inside the voxel, credited where the forward's midpoint rule maps it
+// there, or 0.  in/out: entry and exit plane parameters, of x and y together
+// and of z.
+__device__ __forceinline__ float matched_length(float inxy, float outxy, float inz, float outz, const SidAxis& ax,
+                                                const SidAxis& ay, const SidAxis& az, int ix, int iy, int iz, bool dz_one)
 {
-    const float ain = fmaxf(fmaxf(inx, iny), inz), aout = fminf(fminf(outx, outy), outz);
+    const float ain = fmaxf(inxy, inz), aout = fminf(outxy, outz);
     const float m = (ain + aout) * 0.5f;
     // (every test evaluated: no short-circuit branches)
     const int hit = int(aout > ain) & int(sid_cell_xy(ax, m) == ix) & int(sid_cell_xy(ay, m) == iy) &
                     int(sid_cell_z(az, m, dz_one) == iz);
-    return hit ? (aout - ain) * L : 0.0f;
+    return hit ? aout - ain : 0.0f;
 }
 
 namespace {
-constexpr int MF_A = 48;   // footprint columns in LDS
-constexpr int MF_B = 32;   // footprint rows
+constexpr int MF_A = 48;     // footprint columns in LDS
+constexpr int MF_B = 64;     // footprint rows
+constexpr int MF_W = 2048;   // footprint cells, a column's padded to an odd count
 static_assert(MF_A <= 64 && MF_B <= 64, "footprint columns / rows are staged by one wave each");
 
-// wave-wide min / max (DPP row shifts and lane reads, no LDS round trips);
-// called with every lane of the wave active
-__device__ __forceinline__ int mwave_min(int v) { return __ockl_wfred_min_i32(v); }
-__device__ __forceinline__ int mwave_max(int v) { return __ockl_wfred_max_i32(v); }
+// What a group of four waves stages of a view: per footprint column the plane
+// parameters of its brick's nine x and y planes, per row the entry and exit
+// parameters of each slice's z planes, per cell ray length times sinogram value
+// (column by column; zeros for a column that is none).  What the tables are
+// formed from is double-buffered: written a view ahead.
+template <int BZ>
+struct MatchedLds {
+    float ax[MF_A][9], ay[MF_A][9];
+    float2 zio[MF_B][BZ];
+    float w[MF_W], zero[MF_B];
+    float dx[2][MF_A], dy[2][MF_A], rx[2][MF_A], ry[2][MF_A], dxy2[2][MF_A], tc[2][MF_A];
+    float dz[2][MF_B], rz[2][MF_B], dz2[2][MF_B], tz[2][MF_B];
+    ShadowCols cols[2][64];
+};
 }  // namespace
 
-// 3D, footprint-staged, z-column form: a workgroup is an 8 x 8 x (4*KZ)
-// voxel brick and each thread owns KZ z-adjacent voxels of one (x, y)
-// column.  Per view the workgroup stages in LDS the plane parameters of its
-// nine x planes and nine y planes for each footprint column, and for each
-// footprint row the entry and exit parameters of each of its 4*KZ slices'
-// z planes (each the forward's IEEE division, done once per workgroup),
-// the ray lengths |d| and the sinogram values; each
-// voxel then visits only the cells of its own shadow (the shadow of its
-// column is shared by the four waves through LDS).  Views of each frame in
-// order, columns outer; FP32 accumulation, one fused multiply-add per term.
-// Five workgroups per CU (measured optimum of the register budget).
-template <typename YT, typename XT, int KZ, bool DZ1>
-__global__ __launch_bounds__(256, FL_MATCHED_WG_PER_CU) void k_adj_matched_cone(const YT* __restrict__ Y, XT* __restrict__ X,
-                                                         FwdGeom f, AdjGeom g)
+// 3D, footprint-staged, z-column form: a workgroup is an 8 x 8 x 16 voxel
+// brick, and each thread of a group of four waves owns four z-adjacent voxels
+// of one (x, y) column.  Per view the group stages its footprint (MatchedLds;
+// each plane parameter the forward's IEEE quotient, formed once per group);
+// each voxel then visits the cells of its own shadow, two or three columns of a
+// row at a time.
+//
+// The segment of a (ray, voxel) pair is the smallest of four differences of
+// plane parameters: between the column's slab interval (kept in registers) and
+// the slice's (read per row) both ways, and of either itself.  Where it is
+// longer than tau the forward's midpoint rule credits the voxel (the argument
+// in fl_walk.h: tau = 1.01 2^-23 (4 A + w/|d|), the largest over the axes), and
+// where it is below -tau there is none; only what lies between takes the rule
+// itself.  A z difference far larger than the segment cannot upset the rule
+// along z, so the test is on the differences that involve z planes, and a
+// column whose own interval is that short sends its rows there outright.
+//
+// VG groups share a brick's views between them and add their sums in group
+// order.
+//
+// Bound by VALU issue (some 120 instructions a voxel and view at 256^3: 1.8 rows
+// of 2.3 columns at 20, the rows' ranges 20, the column's slab 9, the rest the
+// tables) and by the waits between its two barriers a view.  256^3, 360 views x
+// 512 x 384: 28.6 -> 21.4 ms; 128^3, 180 views: 2.13 -> 1.45 ms; 64^3, 60 views:
+// 276 -> 81 us; helix 180 x 156 x 132, 241 views x 301 x 217: 15.3 -> 4.0 ms
+// (before: four cell tests per pair, with a division where dz != 1, tables of
+// 32 rows, four slices and one group throughout).  Four waves per SIMD; three
+// (no spills) take 23.7 ms at 256^3.
+template <typename YT, typename XT, int KZ, int VG, bool DZ1>
+__global__ __launch_bounds__(256 * VG, 4) void k_adj_matched_cone(
+    const YT* __restrict__ Y, XT* __restrict__ X, FwdGeom f, AdjGeom g)
 {
     constexpr int BZ = 4 * KZ;
-    __shared__ float t_ax[MF_A][9], t_ay[MF_A][9];
-    __shared__ float t_dx[MF_A], t_dy[MF_A], t_rx[MF_A], t_ry[MF_A], t_dxy2[MF_A];
-    __shared__ float2 t_zio[MF_B][BZ];   // per row and brick slice: z entry / exit plane parameters
-    __shared__ float t_dz[MF_B], t_rz[MF_B], t_dz2[MF_B];
-    __shared__ float t_L[MF_A * MF_B], t_y[MF_A * MF_B];
-    __shared__ int red[2][4][4];
+    constexpr int NY = 2;   // values a thread loads a view ahead
+    __shared__ __align__(16) MatchedLds<BZ> s_lds[VG];
 
     const int bx = (f.nx + 7) / 8, by = (f.ny + 7) / 8, bz = (f.nz + BZ - 1) / BZ;
     const uint32_t nblk = (uint32_t)bx * by * bz;
     const uint32_t b = fl_xcd_remap(blockIdx.x, nblk);
     const int it = blockIdx.y;
-    const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+    const int grp = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 8);
+    const int tid = threadIdx.x & 255, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+    MatchedLds<BZ>& t = s_lds[grp];
     const int ix0 = (int)(b % bx) * 8, iy0 = (int)((b / bx) % by) * 8, iz0 = (int)(b / ((uint32_t)bx * by)) * BZ;
     const int lx = tid & 7, ly = (tid >> 3) & 7, lz0 = wv * KZ;
     const int ix = ix0 + lx, iy = iy0 + ly;
     const bool col = ix < f.nx && iy < f.ny;
+    const int kn = min(KZ, f.nz - iz0 - lz0);   // slices of this wave inside the volume
 
     const int na = f.na, nb = f.nb;
     const float SD = f.SO + f.OD;
     const float xc = (float)ix + 0.5f - (float)(f.nx / 2);
     const float yc = (float)iy + 0.5f - (float)(f.ny / 2);
-    const float hz = 0.5f * f.dz0;
     const ShadowMap ma = fl_shadow_map(f.ya0, f.inv_pa, 0.05f), mb = fl_shadow_map(f.zb0, f.inv_pb, 0.05f);
-    // DZ1: z planes one voxel apart, so the z cell index needs no division
-    // (a compile-time choice: a runtime flag lets the divide be speculated)
+    const float klo = mb.klo + 1.0f, khi = mb.khi;   // floor(k + 1) for ceil(k): the margin covers whole k
+    const bool up = f.inv_pb > 0;
+    const float z0 = (float)(iz0 + lz0 - f.nz / 2);
+    // z planes one voxel apart: the z cell index needs no division (a
+    // compile-time choice: a runtime flag lets the divide be speculated)
     constexpr bool dz_one = DZ1;
+    // tau's constants (fl_walk.h): plane parameters reach at most A here
+    const float rc = 0.5f * sqrtf((float)f.nx * f.nx + (float)f.ny * f.ny);
+    const float A4 = 4.0f * 1.01f * (f.SO + rc + 1.0f) / SD;
+    const float wx = 1.5f * (float)f.nx + 3.0f, wy = 1.5f * (float)f.ny + 3.0f;
+    const float wz = DZ1 ? 1.5f * (float)f.nz + 3.0f : f.dz0 * (2.5f * (float)f.nz + 5.0f);
     float acc[KZ];
 #pragma unroll
     for (int k = 0; k < KZ; k++) acc[k] = 0.0f;
-    const int nvf = g.Nv[it];
-    // The shadow of a thread's (x, y) column is the same in all four waves
-    // (lane -> column is wave-independent): one wave per view computes it a
-    // view ahead, in turn, into double-buffered LDS, written before and read
-    // after the view's first barrier.
-    __shared__ __align__(16) ShadowCols s_cols[2][64];
-    auto col_shadow = [&](int jj) {
-        const int ivv = g.id_Y[it * g.tmp_size + jj];
-        return fl_shadow_cols(f.cs[ivv], f.sn[ivv], f.SO, SD, xc, yc, ma, na);
-    };
-    if (wv == 0 && nvf > 0) s_cols[0][lane] = col_shadow(0);
-    __syncthreads();
-    for (int j = 0; j < nvf; j++) {
+    if (tid < MF_B) t.zero[tid] = 0.0f;
+
+    // The group's views are its own 0, 1, ...: own view i is view i * VG + grp
+    // of the frame's list; 64 of them at a time are set up one per lane: source
+    // and direction, sinogram slot and the brick's footprint on the panel.
+    const int nvf = g.Nv[it], nown = (nvf - grp + VG - 1) / VG, ntrip = (nvf + VG - 1) / VG;
+    float uc = 0.0f, us = 0.0f, usz = 0.0f;
+    int uslot = 0, ua = 0, uan = 0, ub = 0, ubn = 0;   // first column and row and their counts
+    auto setup = [&](int i) {
+        const int j = min((i + lane) * VG + grp, nvf - 1);
         const int iv = g.id_Y[it * g.tmp_size + j];
-        const YT* __restrict__ y = Y + (size_t)g.id_S[it * g.tmp_size + j] * g.nd;
-        const float c = f.cs[iv], s = f.sn[iv];
-        const float sz = f.sdz[iv];
-        int alo = na, ahi = -1, ublo = nb, ubhi = -1;
-        int blo[KZ], bhi[KZ];
+        uslot = g.id_S[it * g.tmp_size + j];
+        uc = f.cs[iv];
+        us = f.sn[iv];
+        usz = f.sdz[iv];
+        // the brick, a hundredth of a voxel wider, and a tenth of a cell
+        const float xm = (float)(ix0 + 4 - f.nx / 2), ym = (float)(iy0 + 4 - f.ny / 2);
+        const float e = 4.01f * (fabsf(uc) + fabsf(us));
+        const float D = uc * xm + us * ym + f.SO, yr = uc * ym - us * xm;
+        const float rn = __builtin_amdgcn_rcpf(D - e) * SD, rf = __builtin_amdgcn_rcpf(D + e) * SD;
+        const float zl = ((float)(iz0 - f.nz / 2) - 0.01f) * f.dz0 - usz;
+        const float zh = ((float)(iz0 + BZ - f.nz / 2) + 0.01f) * f.dz0 - usz;
+        const float yl = yr - e, yh = yr + e;
+        const ShadowMap wa = fl_shadow_map(f.ya0, f.inv_pa, 0.15f), wb = fl_shadow_map(f.zb0, f.inv_pb, 0.15f);
+        int a1, b1;
+        fl_shadow_range(wa, yl * (yl > 0 ? rf : rn), yh * (yh > 0 ? rn : rf), na, ua, a1);
+        fl_shadow_range(wb, zl * (zl > 0 ? rf : rn), zh * (zh > 0 ? rn : rf), nb, ub, b1);
+        if (!(D - e > 0.01f)) {   // a brick that reaches past the source, outside the volume
+            ua = ub = 0;
+            a1 = na - 1;
+            b1 = nb - 1;
+        }
+        uan = max(a1 - ua + 1, 0);
+        ubn = max(b1 - ub + 1, 0);
+    };
+    struct View {
+        float c, s, sz;
+        int A0, nA, B0, nB;
+        size_t off;
+        bool any, fits;
+    };
+    auto lanef = [](float v, int l) { return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), l)); };
+    auto view = [&](int i) {
+        const int l = i & 63;
+        View v;
+        v.c = lanef(uc, l);
+        v.s = lanef(us, l);
+        v.sz = lanef(usz, l);
+        v.A0 = __builtin_amdgcn_readlane(ua, l);
+        v.nA = __builtin_amdgcn_readlane(uan, l);
+        v.B0 = __builtin_amdgcn_readlane(ub, l);
+        v.nB = __builtin_amdgcn_readlane(ubn, l);
+        v.off = (size_t)__builtin_amdgcn_readlane(uslot, l) * g.nd;
+        v.any = i < nown && v.nA > 0 && v.nB > 0;
+        v.fits = v.nA <= MF_A && v.nB <= MF_B && v.nA * (v.nB | 1) <= MF_W;
+        return v;
+    };
+    // a view ahead: direction components, their reciprocals and taus of the
+    // columns (wave 0) and rows (wave 1), the shadows of the thread columns (the
+    // same in all four waves: the other two, in turn) and the cells' values
+    float yv[NY];
+    auto stage = [&](const View& v, int p) {
+        if (!v.any) return;
+        if (v.fits) {
+            if (wv == 0 && lane < v.nA) {
+                const float x1 = v.c * (-f.SO), y1 = v.s * (-f.SO), yd = f.ydet[v.A0 + lane];
+                const float dx = (v.c * f.OD - v.s * yd) - x1, dy = (v.s * f.OD + v.c * yd) - y1;
+                const float rx = 1.0f / dx, ry = 1.0f / dy;
+                t.dx[p][lane] = dx;
+                t.dy[p][lane] = dy;
+                t.rx[p][lane] = rx;
+                t.ry[p][lane] = ry;
+                t.dxy2[p][lane] = dx * dx + dy * dy;   // the first two terms of |d|^2, summed as the forward sums them
+                t.tc[p][lane] = 1.01f * 0x1p-23f * (A4 + fmaxf(wx * fabsf(rx), wy * fabsf(ry)));
+            }
+            if (wv == 1 && lane < v.nB) {
+                const float dz = (f.zdet[v.B0 + lane] + v.sz) - v.sz;
+                const float rz = 1.0f / dz;
+                t.dz[p][lane] = dz;
+                t.rz[p][lane] = rz;
+                t.dz2[p][lane] = dz * dz;
+                t.tz[p][lane] = 1.01f * 0x1p-23f * (wz * fabsf(rz));
+            }
+            const uint32_t mA = fl_small_div_m((uint32_t)v.nA);   // k * nA < 2^18 in these tables
+            const YT* __restrict__ y = Y + v.off + (size_t)v.B0 * na + v.A0;
 #pragma unroll
-        for (int k = 0; k < KZ; k++) { blo[k] = nb; bhi[k] = -1; }
-        const ShadowCols sc = s_cols[j & 1][lane];
-        if (wv == (j & 3) && j + 1 < nvf) s_cols[(j + 1) & 1][lane] = col_shadow(j + 1);
-        if (col) {
-            alo = sc.alo;
-            ahi = sc.ahi;
-#pragma unroll
-            for (int k = 0; k < KZ; k++) {
-                const int iz = iz0 + lz0 + k;
-                if (iz < f.nz && alo <= ahi) {
-                    const float zc = ((float)iz + 0.5f - (float)(f.nz / 2)) * f.dz0;
-                    int bl, bh;
-                    fl_shadow_rows(sc, zc - sz, hz, mb, nb, bl, bh);
-                    if (bl <= bh) {
-                        blo[k] = bl; bhi[k] = bh;
-                        ublo = min(ublo, bl); ubhi = max(ubhi, bh);
-                    }
+            for (int q = 0; q < NY; q++) {
+                const int k = q * 256 + tid;
+                if (k < v.nA * v.nB) {
+                    const int kb = fl_small_div(k, mA), ka = k - __mul24(kb, v.nA);
+                    yv[q] = fl_load(y, (size_t)((unsigned)kb * (unsigned)na + (unsigned)ka));
                 }
             }
-            if (ubhi < 0) { alo = na; ahi = -1; }
         }
-        {
-            int m0 = mwave_min(alo), m1 = mwave_max(ahi), m2 = mwave_min(ublo), m3 = mwave_max(ubhi);
-            if (lane == 0) {
-                red[j & 1][wv][0] = m0; red[j & 1][wv][1] = m1;
-                red[j & 1][wv][2] = m2; red[j & 1][wv][3] = m3;
+        if (wv == 2 + p) t.cols[p][lane] = fl_shadow_cols(v.c, v.s, f.SO, SD, xc, yc, ma, na);
+    };
+    View v{};
+    int p = 0;   // the buffer of the staged view
+    if (nvf > 0) {
+        setup(0);
+        v = view(0);
+        stage(v, 0);
+    }
+    for (int i = 0; i < ntrip; i++) {
+        if (VG == 1 && !v.any) {   // the brick is off the panel; the other buffer may be in use
+            if (i + 1 < ntrip) {
+                if ((i + 1) % 64 == 0) setup(i + 1);
+                v = view(i + 1);
+                stage(v, p);
             }
+            continue;
         }
+        const bool staged = v.any && v.fits;
+        const float x1 = v.c * (-f.SO), y1 = v.s * (-f.SO), z1 = v.sz;
         __syncthreads();
-        int A0 = red[j & 1][0][0], A1 = red[j & 1][0][1], B0 = red[j & 1][0][2], B1 = red[j & 1][0][3];
-#pragma unroll
-        for (int w = 1; w < 4; w++) {
-            A0 = min(A0, red[j & 1][w][0]); A1 = max(A1, red[j & 1][w][1]);
-            B0 = min(B0, red[j & 1][w][2]); B1 = max(B1, red[j & 1][w][3]);
-        }
-        const int nA = A1 - A0 + 1, nB = B1 - B0 + 1;
-        if (nA <= 0 || nB <= 0) continue;
-        const float x1 = c * (-f.SO), y1 = s * (-f.SO), z1 = sz;
-        if (nA <= MF_A && nB <= MF_B) {
-            // columns (wave 0): direction components; rows (wave 1) likewise;
-            // both fit one wave, and their load and divide latencies overlap
-            if (tid < nA) {
-                const int k = tid;
-                const float yd = f.ydet[A0 + k];
-                const float dx = (c * f.OD - s * yd) - x1, dy = (s * f.OD + c * yd) - y1;
-                t_dx[k] = dx; t_dy[k] = dy;
-                t_dxy2[k] = dx * dx + dy * dy;   // the first two terms of |d|^2, summed as the forward sums them
-                t_rx[k] = 1.0f / dx; t_ry[k] = 1.0f / dy;
-            }
-            if (tid >= 64 && tid - 64 < nB) {
-                const int k = tid - 64;
-                const float dz = (f.zdet[B0 + k] + sz) - z1;
-                t_dz[k] = dz;
-                t_dz2[k] = dz * dz;
-                t_rz[k] = 1.0f / dz;
-            }
-            __syncthreads();
+        if (staged) {
             // plane coordinate i -> ((float)i - o)/d, the forward's IEEE
             // quotient, from the staged reciprocal of d
-            for (int k = tid; k < nA * 9; k += 256) {
-                const int ka = k / 9, q = k % 9;
-                t_ax[ka][q] = fl_div_r((float)(ix0 + q - f.nx / 2) - x1, t_dx[ka], t_rx[ka]);
-                t_ay[ka][q] = fl_div_r((float)(iy0 + q - f.ny / 2) - y1, t_dy[ka], t_ry[ka]);
+            if ((tid & 15) < 9) {
+                const int q = tid & 15;
+                const float nx = (float)(ix0 + q - f.nx / 2) - x1, ny = (float)(iy0 + q - f.ny / 2) - y1;
+                for (int ka = tid >> 4; ka < v.nA; ka += 16) {
+                    t.ax[ka][q] = sid_div(nx, t.dx[p][ka], t.rx[p][ka]);
+                    t.ay[ka][q] = sid_div(ny, t.dy[p][ka], t.ry[p][ka]);
+                }
             }
             // per row and brick slice the parameters of the slice's two z
             // planes (the forward's quotients), ordered as entry and exit
             // along the ray (+-inf for a ray parallel to them)
-            for (int k = tid; k < nB * BZ; k += 256) {
-                const int kb = k / BZ, q = k % BZ;
-                const float dz = t_dz[kb], rz = t_rz[kb];
-                const float lo = fl_div_r((float)(iz0 + q - f.nz / 2) * f.dz0 - z1, dz, rz);
-                const float hi = fl_div_r((float)(iz0 + q + 1 - f.nz / 2) * f.dz0 - z1, dz, rz);
-                t_zio[kb][q] = dz != 0.0f ? make_float2(dz > 0 ? lo : hi, dz > 0 ? hi : lo)
-                                          : make_float2(-FL_INF, FL_INF);
-            }
-            const uint32_t mA = fl_small_div_m((uint32_t)nA);   // k * nA < 2^18 in these tables
-            for (int k = tid; k < nA * nB; k += 256) {
-                const int kb = fl_small_div(k, mA), ka = k - kb * nA;
-                // |d| = sqrtf(dx*dx + dy*dy + dz*dz), the forward's ray length
-                // bit for bit (left-to-right sum, correctly rounded root)
-                t_L[k] = sqrtf(t_dxy2[ka] + t_dz2[kb]);
-                t_y[k] = fl_load(y, (size_t)(B0 + kb) * na + (A0 + ka));
-            }
-            __syncthreads();
-            // columns outermost (no reference order to keep): the column's x/y
-            // slab interval is formed once and serves every row and voxel
-            for (int ia = alo; ia <= ahi; ia++) {
-                const int ka = ia - A0;
-                const float dx = t_dx[ka], dy = t_dy[ka];
-                SidAxis ax, ay;
-                sid_axis_init(ax, x1, dx, 1.0f, f.nx);
-                sid_axis_init(ay, y1, dy, 1.0f, f.ny);
-                const float x_lo = t_ax[ka][lx], x_hi = t_ax[ka][lx + 1];
-                const float y_lo = t_ay[ka][ly], y_hi = t_ay[ka][ly + 1];
-                const float inx = ax.on ? (dx > 0 ? x_lo : x_hi) : -FL_INF;
-                const float outx = ax.on ? (dx > 0 ? x_hi : x_lo) : FL_INF;
-                const float iny = ay.on ? (dy > 0 ? y_lo : y_hi) : -FL_INF;
-                const float outy = ay.on ? (dy > 0 ? y_hi : y_lo) : FL_INF;
-                if (!(fminf(outx, outy) > fmaxf(inx, iny))) continue;   // misses the (x, y) column
-#pragma unroll
-                for (int k = 0; k < KZ; k++) {
-                    const int lz = lz0 + k, iz = iz0 + lz;
-                    for (int ib = blo[k]; ib <= bhi[k]; ib++) {
-                        const int kb = ib - B0;
-                        const float dz = t_dz[kb];
-                        SidAxis az;
-                        sid_axis_init(az, z1, dz, f.dz0, f.nz);
-                        const float2 zio = t_zio[kb][lz];
-                        const float inz = zio.x, outz = zio.y;
-                        const int q = kb * nA + ka;
-                        const float Si = matched_coef(inx, outx, iny, outy, inz, outz, ax, ay, az, ix, iy, iz,
-                                                      dz_one, t_L[q]);
-                        // one fused multiply-add (no reference rounding to keep;
-                        // +-0 for a miss leaves the sum unchanged)
-                        acc[k] = __builtin_fmaf(Si, t_y[q], acc[k]);
-                    }
+            {
+                const int q = tid % BZ;
+                const float n0 = (float)(iz0 + q - f.nz / 2) * f.dz0 - z1, n1 = (float)(iz0 + q + 1 - f.nz / 2) * f.dz0 - z1;
+                for (int kb = tid / BZ; kb < v.nB; kb += 256 / BZ) {
+                    const float dz = t.dz[p][kb], rz = t.rz[p][kb];
+                    const float lo = sid_div(n0, dz, rz), hi = sid_div(n1, dz, rz);
+                    t.zio[kb][q] = dz != 0.0f ? make_float2(fminf(lo, hi), fmaxf(lo, hi)) : make_float2(-FL_INF, FL_INF);
                 }
             }
-        } else if (alo <= ahi) {
+            // |d| = sqrtf(dx*dx + dy*dy + dz*dz), the forward's ray length
+            // (left-to-right sum, correctly rounded root), times the value
+            const uint32_t mA = fl_small_div_m((uint32_t)v.nA);
+            auto put = [&](int k, float yk) {
+                const int kb = fl_small_div(k, mA), ka = k - __mul24(kb, v.nA);
+                t.w[__mul24(ka, v.nB | 1) + kb] = fl_sqrt_nonneg(t.dxy2[p][ka] + t.dz2[p][kb]) * yk;
+            };
+            const int cells = v.nA * v.nB;
+#pragma unroll
+            for (int q = 0; q < NY; q++)
+                if (q * 256 + tid < cells) put(q * 256 + tid, yv[q]);
+            for (int k = NY * 256 + tid; k < cells; k += 256) {
+                const int kb = fl_small_div(k, mA), ka = k - __mul24(kb, v.nA);
+                put(k, fl_load(Y + v.off, (size_t)(v.B0 + kb) * na + (v.A0 + ka)));
+            }
+        }
+        const View u = v;
+        if (i + 1 < ntrip) {
+            if ((i + 1) % 64 == 0) setup(i + 1);
+            v = view(i + 1);
+        }
+        __syncthreads();
+        const int p0 = p;
+        p ^= 1;
+        if (i + 1 < ntrip) stage(v, p);
+        const ShadowCols sc = t.cols[p0][lane];
+        if (!u.any || !col || sc.alo > sc.ahi) continue;
+        // rows of slice k, from its edges' projections at the column's near and
+        // far ends (e: the lower edge's, handed on to the next slice)
+        const float rn = sc.rn * mb.inv_p, rf = sc.rf * mb.inv_p;
+        struct Edge {
+            float lo, hi;
+        };
+        auto edge = [&](int k) {
+            const float e = (z0 + (float)k) * f.dz0 - u.sz;
+            return Edge{fminf(e * rn, e * rf), fmaxf(e * rn, e * rf)};
+        };
+        const float kl = klo - (float)u.B0, kh = khi - (float)u.B0;
+        auto rows = [&](Edge& e, int k, int& blo, int& bhi) {
+            const Edge e1 = edge(k + 1);
+            blo = max(sid_floor((up ? e.lo : e1.lo) + kl), 0);
+            bhi = min(sid_floor((up ? e1.hi : e.hi) + kh), u.nB - 1);
+            e = e1;
+        };
+        if (staged) {
+            const int alo = max(sc.alo, u.A0) - u.A0, ahi = min(sc.ahi, u.A0 + u.nA - 1) - u.A0;
+            const int wst = u.nB | 1;
+            // CA columns from a on
+            auto part = [&](auto ca, int a) {
+                constexpr int CA = decltype(ca)::value;
+                float ixy[CA], oxy[CA], dxy[CA], thc = 0.0f;
+                const float* wp[CA];
+#pragma unroll
+                for (int c = 0; c < CA; c++) {
+                    const int ka = min(a + c, ahi);
+                    const float x0 = t.ax[ka][lx], x2 = t.ax[ka][lx + 1], y0 = t.ay[ka][ly], y2 = t.ay[ka][ly + 1];
+                    const float tc = t.tc[p0][ka];
+                    float inx = fminf(x0, x2), outx = fmaxf(x0, x2), iny = fminf(y0, y2), outy = fmaxf(y0, y2);
+                    if (!(tc < FL_INF)) {   // parallel to an axis's planes: the rule decides
+                        if (t.dx[p0][ka] == 0.0f) { inx = -FL_INF; outx = FL_INF; }
+                        if (t.dy[p0][ka] == 0.0f) { iny = -FL_INF; outy = FL_INF; }
+                    }
+                    ixy[c] = fmaxf(inx, iny);
+                    oxy[c] = fminf(outx, outy);
+                    dxy[c] = oxy[c] - ixy[c];
+                    wp[c] = &t.w[__mul24(ka, wst)];
+                    if (a + c <= ahi && dxy[c] > 0.0f) {
+                        thc = fmaxf(thc, dxy[c] > tc ? tc : FL_INF);
+                    } else {   // misses the (x, y) column: nothing, whatever its values
+                        ixy[c] = -1e30f;
+                        oxy[c] = 1e30f;
+                        dxy[c] = -1.0f;
+                        wp[c] = t.zero;
+                    }
+                }
+                Edge e = edge(0);
+#pragma unroll
+                for (int k = 0; k < KZ; k++) {
+                    if (k >= kn) break;
+                    int blo, bhi;
+                    rows(e, k, blo, bhi);
+                    for (int kb = blo; kb <= bhi; kb++) {
+                        const float2 zio = t.zio[kb][lz0 + k];
+                        const float th = thc + t.tz[p0][kb], dzz = zio.y - zio.x;
+                        float w[CA], l[CA], near = dzz;
+#pragma unroll
+                        for (int c = 0; c < CA; c++) w[c] = wp[c][kb];
+#pragma unroll
+                        for (int c = 0; c < CA; c++) {
+                            const float d1 = oxy[c] - zio.x, d2 = zio.y - ixy[c];
+                            near = fminf(near, fminf(fabsf(d1), fabsf(d2)));
+                            l[c] = __builtin_amdgcn_fmed3f(fminf(fminf(d1, d2), dxy[c]), 0.0f, dzz);
+                        }
+                        if (near <= th) {
+                            SidAxis ax, ay, az;
+                            sid_axis_init(az, z1, t.dz[p0][kb], f.dz0, f.nz);
+#pragma unroll
+                            for (int c = 0; c < CA; c++) {
+                                if (dxy[c] <= 0.0f) continue;
+                                const int ka = a + c;
+                                sid_axis_init(ax, x1, t.dx[p0][ka], 1.0f, f.nx);
+                                sid_axis_init(ay, y1, t.dy[p0][ka], 1.0f, f.ny);
+                                l[c] = matched_length(ixy[c], oxy[c], zio.x, zio.y, ax, ay, az, ix, iy, iz0 + lz0 + k, dz_one);
+                            }
+                        }
+#pragma unroll
+                        for (int c = 0; c < CA; c++) acc[k] = __builtin_fmaf(l[c], w[c], acc[k]);
+                    }
+                }
+            };
+            // two columns or three, whichever the wave needs
+            for (int a = alo; a <= ahi;) {
+                if (__builtin_amdgcn_ballot_w64(a + 1 < ahi) == 0) {
+                    part(std::integral_constant<int, 2>{}, a);
+                    a += 2;
+                } else {
+                    part(std::integral_constant<int, 3>{}, a);
+                    a += 3;
+                }
+            }
+        } else {
+            const YT* __restrict__ y = Y + u.off;
+            Edge e = edge(0);
 #pragma unroll
             for (int k = 0; k < KZ; k++) {
+                if (k >= kn) break;
                 const int iz = iz0 + lz0 + k;
-                for (int ib = blo[k]; ib <= bhi[k]; ib++) {
-                    const float dz = (f.zdet[ib] + sz) - z1;
+                int blo, bhi;
+                rows(e, k, blo, bhi);
+                for (int ib = blo + u.B0; ib <= bhi + u.B0; ib++) {
+                    const float dz = (f.zdet[ib] + u.sz) - z1;
                     SidAxis az;
                     sid_axis_init(az, z1, dz, f.dz0, f.nz);
                     const FlAxisIv sv = fl_slab_r(az, iz, 1.0f / dz);
-                    for (int ia = alo; ia <= ahi; ia++) {
+                    for (int ia = max(sc.alo, u.A0); ia <= min(sc.ahi, u.A0 + u.nA - 1); ia++) {
                         const float yd = f.ydet[ia];
-                        const float dx = (c * f.OD - s * yd) - x1, dy = (s * f.OD + c * yd) - y1;
+                        const float dx = (u.c * f.OD - u.s * yd) - x1, dy = (u.s * f.OD + u.c * yd) - y1;
                         SidAxis ax, ay;
                         sid_axis_init(ax, x1, dx, 1.0f, f.nx);
                         sid_axis_init(ay, y1, dy, 1.0f, f.ny);
                         const FlAxisIv sx = fl_slab_r(ax, ix, 1.0f / dx), sy = fl_slab_r(ay, iy, 1.0f / dy);
-                        const float L = sqrtf(dx * dx + dy * dy + dz * dz);
-                        const float Si = matched_coef(sx.in, sx.out, sy.in, sy.out, sv.in, sv.out, ax, ay, az, ix,
-                                                      iy, iz, dz_one, L);
+                        const float len = matched_length(fmaxf(sx.in, sy.in), fminf(sx.out, sy.out), sv.in, sv.out, ax, ay,
+                                                         az, ix, iy, iz, dz_one);
+                        const float Si = len * sqrtf(dx * dx + dy * dy + dz * dz);
                         if (Si != 0.0f) acc[k] = __builtin_fmaf(Si, fl_load(y, (size_t)ib * na + ia), acc[k]);
                     }
                 }
             }
         }
+    }
+    if constexpr (VG > 1) {
+        // the groups' sums, in group order
+        __syncthreads();
+        float* part = (float*)&s_lds[grp];
+#pragma unroll
+        for (int k = 0; k < KZ; k++) part[k * 256 + tid] = acc[k];
+        __syncthreads();
+        if (grp > 0) return;
+#pragma unroll
+        for (int o = 1; o < VG; o++)
+#pragma unroll
+            for (int k = 0; k < KZ; k++) acc[k] = acc[k] + ((const float*)&s_lds[o])[k * 256 + tid];
     }
     if (col) {
 #pragma unroll
@@ -290,19 +452,41 @@ __global__ __launch_bounds__(256) void k_adj_matched_fan(const YT* __restrict__ 
     fl_store(X, (size_t)it * f.nvox + (size_t)iy * f.nx + ix, fl_fan_matched_pixel(Y, f, g, it, ix, iy));
 }
 
+// Rows of the largest footprint of a brick of bz slices.
+static double matched_rows(const FwdGeom& f, int bz)
+{
+    const double rc = 0.5 * sqrt((double)f.nx * f.nx + (double)f.ny * f.ny), SD = (double)f.SO + f.OD;
+    const double near = std::max((double)f.SO - rc, 1.0), zmax = 0.5 * f.nz * f.dz0 + bz * f.dz0;
+    return (bz * f.dz0 * SD / near + zmax * (SD / near - SD / (near + 11.4))) * fabs((double)f.inv_pb) + 3.0;
+}
+
 template <typename YT, typename XT>
 static hipError_t launch_matched_t(const void* Y, void* X, const fl_plan_s* p, hipStream_t st)
 {
     const FwdGeom& f = p->fg;
     if (p->cone) {
-        constexpr int KZ = 4;
-        uint32_t nblk = (uint32_t)((f.nx + 7) / 8) * ((f.ny + 7) / 8) * ((f.nz + 4 * KZ - 1) / (4 * KZ));
-        if (f.dz0 == 1.0f)
-            hipLaunchKernelGGL((k_adj_matched_cone<YT, XT, KZ, true>), dim3(nblk, p->nt), dim3(256), 0, st,
-                               (const YT*)Y, (XT*)X, f, p->ag);
-        else
-            hipLaunchKernelGGL((k_adj_matched_cone<YT, XT, KZ, false>), dim3(nblk, p->nt), dim3(256), 0, st,
-                               (const YT*)Y, (XT*)X, f, p->ag);
+        const auto blocks = [&](int kz) { return (uint32_t)((f.nx + 7) / 8) * ((f.ny + 7) / 8) * ((f.nz + 4 * kz - 1) / (4 * kz)); };
+        auto go = [&](auto kz, auto vg) {
+            constexpr int KZ = decltype(kz)::value, VG = decltype(vg)::value;
+            const dim3 grid(blocks(KZ), p->nt), block(256 * VG);
+            if (f.dz0 == 1.0f)
+                hipLaunchKernelGGL((k_adj_matched_cone<YT, XT, KZ, VG, true>), grid, block, 0, st, (const YT*)Y, (XT*)X, f, p->ag);
+            else
+                hipLaunchKernelGGL((k_adj_matched_cone<YT, XT, KZ, VG, false>), grid, block, 0, st, (const YT*)Y, (XT*)X, f, p->ag);
+        };
+        using I8 = std::integral_constant<int, 8>;
+        using I4 = std::integral_constant<int, 4>;
+        using I1 = std::integral_constant<int, 1>;
+        // N^3 voxels, 96 views, us (eight slices a thread, four, four with the
+        // views shared by four groups): 48^3 536, 319, 125; 80^3 585, 349, 245;
+        // 96^3 614, 435, 473; 112^3 727, 689, 705; 120^3 743, 815, 921; 128^3
+        // 759, 839, 961.  Four groups pay while a CU has at most two such
+        // workgroups to run, eight slices once it has three or more.  A finely
+        // sampled panel keeps to four slices (helix 180 x 156 x 132, rows 0.36
+        // slices apart: 4.0 ms, 18.5 ms where the rows overflow the tables).
+        if (blocks(4) * (size_t)p->nt <= 512) go(I4{}, I4{});
+        else if (blocks(8) * (size_t)p->nt >= 768 && matched_rows(f, 32) <= MF_B) go(I8{}, I1{});
+        else go(I4{}, I1{});
     } else {
         dim3 grid((f.nx + 15) / 16, (f.ny + 15) / 16, p->nt);
         if (!fl_launch_fan_adj_w<FanMatched>((const YT*)Y, (XT*)X, f, p->ag, st))
