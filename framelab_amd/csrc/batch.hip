@@ -69,22 +69,23 @@ __global__ __launch_bounds__(64) void k_bfwd(const float* __restrict__ X, float*
         const FwdGeom f = D[p].f;
         const int local = item - start[p];
         const int tc = T / FV, tpv = (f.na + tc - 1) / tc;
-        const int slot = local / tpv * FV + (int)threadIdx.x / FAN_WA, t = local % tpv;
-        const int iv = f.slot_view[min(slot, f.nslots - 1)];
-        const float* x = X + D[p].voff + (size_t)f.view_frame[iv] * f.nvox;
-        float* y = Y + D[p].soff + (size_t)slot * f.na;
-        for (int k = 0; k < tc; k += FAN_WA) {
-            const int id = t * tc + k + (int)threadIdx.x % FAN_WA;
-            const bool live = slot < f.nslots && id < f.na;
-            float v = 0.0f;
-            if (GAO) {
-                if (live) v = fl_fan_gao_sum(x, f, iv, id);
-            } else if (fl_fan_small(f.nx, f.ny)) {
-                v = fl_fan_ray_sum<true>(x, f, iv, min(id, f.na - 1), live);
-            } else {
-                v = fl_fan_ray_sum<false>(x, f, iv, min(id, f.na - 1), live);
+        const int t = local % tpv;
+        constexpr int WA = GAO ? GAO_WA : FAN_WA, WV = (GAO ? 16 : 64) / WA;   // a wave's cells and views
+        const int ray = GAO ? (int)threadIdx.x / 4 : (int)threadIdx.x;
+        float* y = Y + D[p].soff;
+        for (int sv = 0; sv < FV; sv += WV) {
+            const int slot = local / tpv * FV + sv + ray / WA;
+            const int iv = f.slot_view[min(slot, f.nslots - 1)];
+            const float* x = X + D[p].voff + (size_t)f.view_frame[iv] * f.nvox;
+            for (int k = 0; k < tc; k += WA) {
+                const int id = t * tc + k + ray % WA;
+                const bool live = slot < f.nslots && id < f.na;
+                const int ia = min(id, f.na - 1);
+                float v;
+                if (fl_fan_small(f.nx, f.ny)) v = GAO ? fl_fan_gao_sum<true>(x, f, iv, ia) : fl_fan_ray_sum<true>(x, f, iv, ia, live);
+                else v = GAO ? fl_fan_gao_sum<false>(x, f, iv, ia) : fl_fan_ray_sum<false>(x, f, iv, ia, live);
+                if (live && (!GAO || (threadIdx.x & 3) == 0)) y[(size_t)slot * f.na + id] = v;
             }
-            if (live) y[id] = v;
         }
     }
 }

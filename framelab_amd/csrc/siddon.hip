@@ -388,24 +388,31 @@ hipError_t fl_launch_trace(const FwdGeom& g, int cone, int nrays, const int* ray
 }
 
 // ---- Gao column-walk fan forward (class default, version 1) -------------
-template <typename VT, typename YT>
+// One wave per workgroup: its 16 rays, GAO_WA cells of 16 / GAO_WA views.
+template <typename VT, typename YT, bool SMALL>
 __global__ __launch_bounds__(64) void k_fwd_fan_gao(const VT* __restrict__ X, YT* __restrict__ Y, FwdGeom g)
 {
-    const uint32_t tiles = (g.na + 63) / 64;
+    constexpr int WA = GAO_WA, WV = 16 / WA;
+    const uint32_t tiles = (g.na + WA - 1) / WA;
     const uint32_t b = fl_xcd_remap(blockIdx.x, gridDim.x);
-    const int slot = (int)(b / tiles);
-    const int id = (int)(b % tiles) * 64 + (int)threadIdx.x;
-    if (slot >= g.nslots || id >= g.na) return;
-    const int iv = g.slot_view[slot];
-    fl_store(Y, (size_t)slot * g.na + id, fl_fan_gao_sum(X + (size_t)g.view_frame[iv] * g.nvox, g, iv, id));
+    const int ray = (int)threadIdx.x >> 2;
+    const int slot = (int)(b / tiles) * WV + ray / WA;
+    const int id = (int)(b % tiles) * WA + ray % WA;
+    const int iv = g.slot_view[min(slot, g.nslots - 1)];
+    const float v = fl_fan_gao_sum<SMALL>(X + (size_t)g.view_frame[iv] * g.nvox, g, iv, min(id, g.na - 1));
+    if (slot < g.nslots && id < g.na && (threadIdx.x & 3) == 0) fl_store(Y, (size_t)slot * g.na + id, v);
 }
 
 template <typename VT, typename YT>
 static hipError_t launch_fan_gao_t(const void* X, void* Y, const FwdGeom& g, hipStream_t st)
 {
-    uint32_t grid = ((g.na + 63) / 64) * (uint32_t)g.nslots;
+    constexpr int WV = 16 / GAO_WA;
+    const uint32_t grid = (uint32_t)((g.na + GAO_WA - 1) / GAO_WA) * (uint32_t)((g.nslots + WV - 1) / WV);
     if (grid == 0) return hipSuccess;
-    hipLaunchKernelGGL((k_fwd_fan_gao<VT, YT>), dim3(grid), dim3(64), 0, st, (const VT*)X, (YT*)Y, g);
+    if (fl_fan_small(g.nx, g.ny))
+        hipLaunchKernelGGL((k_fwd_fan_gao<VT, YT, true>), dim3(grid), dim3(64), 0, st, (const VT*)X, (YT*)Y, g);
+    else
+        hipLaunchKernelGGL((k_fwd_fan_gao<VT, YT, false>), dim3(grid), dim3(64), 0, st, (const VT*)X, (YT*)Y, g);
     return hipGetLastError();
 }
 
