@@ -18,9 +18,9 @@
 // produces all NF^d bands from it (separably, in registers), so the input is
 // read once and every band is written once (the transform is write-bound).
 // 3D synthesis runs separably on LDS tiles (k_iwt3m, marching through z,
-// for dilations 1 and 2, k_iwt3s beyond); 2D synthesis, and 3D levels whose
-// halo outgrows the tiles, gather each band's neighbourhood per output.  All accumulate in
-// FP32.
+// for dilations 1 and 2, k_iwt3s beyond), 2D synthesis marches through y
+// (k_iwt2m); levels whose halo outgrows the tiles gather each band's
+// neighbourhood per output.  All accumulate in FP32.
 #include <algorithm>
 #include <type_traits>
 
@@ -462,7 +462,8 @@ __global__ __launch_bounds__(4 * TXW) void k_iwt3m(const CT* __restrict__ C, XT*
 // rows are 256 wide or a multiple of it and their LDS fits 160 KB (no x
 // halo: the taps wrap inside the tile), else 64-wide tiles.  Output slices
 // per workgroup: the longest run (fewer halo re-reads) that still gives at
-// least one workgroup per CU and `min_waves` waves, at least 4.
+// least one workgroup per CU and `min_waves` waves, at least 4; fewer where not
+// even those give a workgroup per CU (64^3, linear: 66 -> 34 us).
 template <int NF, int NT, int STEP, typename CT, typename XT>
 static void launch_iwt3m(const FlFrameDesc& f, const CT* C, XT* u, const FlTaps& T, float alpha, float beta,
                          const float* base, const CT* lp, hipStream_t st)
@@ -474,6 +475,7 @@ static void launch_iwt3m(const FlFrameDesc& f, const CT* C, XT* u, const FlTaps&
         const size_t min_groups = std::max<size_t>(256, (size_t)FL_IWT_MIN_WAVES / (TXW / 16));
         int zs = 64;
         while (zs > 4 && (size_t)tiles * ((f.nz + zs - 1) / zs) < min_groups) zs /= 2;
+        while (zs > 1 && (size_t)tiles * ((f.nz + zs - 1) / zs) < 256) zs /= 2;
         zs = std::min(zs, std::max(f.nz, 1));
         const dim3 grid(tiles * (unsigned)((f.nz + zs - 1) / zs));
         hipLaunchKernelGGL((k_iwt3m<NF, NT, STEP, TXW, CT, XT>), grid, dim3(4 * TXW), 0, st, C, u, f.nx, f.ny, f.nz,
@@ -506,6 +508,7 @@ __global__ __launch_bounds__(256) void k_fwt2(const XT* __restrict__ u, CT* __re
     for (int b = 0; b < NF * NF; b++) fl_store(C, (size_t)b * npix + idx, w[b]);
 }
 
+// 2D synthesis, general form: the bands' neighbourhood gathered per pixel.
 template <int NF, int NT, typename CT, typename XT>
 __global__ __launch_bounds__(256) void k_iwt2(const CT* __restrict__ C, XT* u, int nx, int ny,
                                              int step, FlTaps T, float alpha, float beta,
@@ -518,6 +521,106 @@ __global__ __launch_bounds__(256) void k_iwt2(const CT* __restrict__ C, XT* u, i
     float v = alpha * fl_synth2<NF, NT>(C, npix, nx, ny, x, y, step, T, lp);
     if (base) v = __builtin_fmaf(beta, base[idx], v);
     fl_store(u, idx, v);
+}
+
+// 2D synthesis marching through y, separable: u = sum_i corr_x[R_i] S_i with
+// S_i = sum_j corr_y[R_j] C_ij.  A workgroup of TXW threads owns TXW columns
+// (the outer h = (NT-1)/2 * step on either side are halo) and `rc` output rows
+// `step` apart; a thread walks its column, adding each coefficient to the NT
+// partial sums it taps (in registers), so a coefficient is read (rc + NT - 1) /
+// rc times; a finished row of S goes through LDS for the x pass.  Bound by
+// reading the coefficients, mostly from cache.  1001 x 777, cubic: 69 -> 27
+// us a level (the general form gathers 625 taps a pixel); 2048 x 2048, linear:
+// 132 -> 42 us.
+// Same in-place contract as k_iwt3.
+template <int NF, int NT, int TXW, typename CT, typename XT>
+__global__ __launch_bounds__(TXW) void k_iwt2m(const CT* __restrict__ C, XT* u, int nx, int ny, int step, int rc,
+                                              FlTaps T, float alpha, float beta, const float* base, const CT* lp)
+{
+    constexpr int CC = (NT - 1) / 2;
+    __shared__ float sx[2][NF][TXW];
+    const int h = CC * step, txo = TXW - 2 * h, tid = threadIdx.x;
+    const size_t npix = (size_t)nx * ny;
+    const int x = (int)blockIdx.x * txo - h + tid, xw = wrapi(x, nx);
+    const int y0 = (int)(blockIdx.y / step) * rc * step + (int)(blockIdx.y % step);   // first output row
+    const int nrow = min(rc, (ny - y0 + step - 1) / step);
+    const bool own = tid >= h && tid < TXW - h && x < nx;
+    const int dy = step % ny;
+    int y = wrapi(y0 - h, ny);
+    float S[NF][NT];   // S[i][m]: output row (row read) - CC + m
+#pragma unroll
+    for (int i = 0; i < NF; i++)
+#pragma unroll
+        for (int m = 0; m < NT; m++) S[i][m] = 0.0f;
+    for (int r = 0; r < nrow + 2 * CC; r++) {
+        const size_t o = (size_t)y * nx + xw;
+        float c[NF][NF];
+#pragma unroll
+        for (int j = 0; j < NF; j++)
+#pragma unroll
+            for (int i = 0; i < NF; i++) c[i][j] = fl_load(band_ptr(C, i + NF * j, npix, lp), o);
+        y += dy;
+        if (y >= ny) y -= ny;
+#pragma unroll
+        for (int i = 0; i < NF; i++)
+#pragma unroll
+            for (int j = 0; j < NF; j++)
+#pragma unroll
+                for (int m = 0; m < NT; m++) S[i][m] = __builtin_fmaf(T.R[j][NT - 1 - m], c[i][j], S[i][m]);
+        if (r >= 2 * CC) {
+            float (&s)[NF][TXW] = sx[r & 1];
+#pragma unroll
+            for (int i = 0; i < NF; i++) s[i][tid] = S[i][0];
+            __syncthreads();
+            if (own) {
+                float v = 0.0f;
+#pragma unroll
+                for (int i = 0; i < NF; i++) {
+                    float a = 0.0f;
+#pragma unroll
+                    for (int kx = 0; kx < NT; kx++) a = __builtin_fmaf(T.R[i][kx], s[i][tid + (kx - CC) * step], a);
+                    v += a;
+                }
+                const size_t idx = (size_t)(y0 + (r - 2 * CC) * step) * nx + x;
+                v = alpha * v;
+                if (base) v = __builtin_fmaf(beta, base[idx], v);
+                fl_store(u, idx, v);
+            }
+        }
+#pragma unroll
+        for (int i = 0; i < NF; i++) {
+#pragma unroll
+            for (int m = 0; m + 1 < NT; m++) S[i][m] = S[i][m + 1];
+            S[i][NT - 1] = 0.0f;
+        }
+    }
+}
+
+// Launch of the 2D synthesis: one-wave tiles while the halo leaves them half
+// their columns, tiles of four waves while it leaves those, the gather beyond.
+// Rows per workgroup: 16, fewer where that leaves under 768 waves (1001 x 777
+// cubic, two levels: 16 rows 28 + 26 us, 8 rows 32 + 28, 4 rows 45 + 37; 512 x
+// 512: alike; 2048 x 2048: 32 rows 119 us, 64 rows 144).
+template <int NF, int NT, typename CT, typename XT>
+static void launch_iwt2(const FlFrameDesc& f, const CT* C, XT* u, int step, const FlTaps& T, float alpha, float beta,
+                        const float* base, const CT* lp, hipStream_t st)
+{
+    const int h = (NT - 1) / 2 * step;
+    auto go = [&](auto txw) {
+        constexpr int TXW = decltype(txw)::value;
+        const unsigned tiles = (unsigned)((f.nx + TXW - 2 * h - 1) / (TXW - 2 * h));
+        auto groups = [&](int rc) { return (size_t)((f.ny + (size_t)rc * step - 1) / ((size_t)rc * step)) * step; };
+        int rc = 16;
+        while (rc > 4 && (size_t)tiles * groups(rc) * (TXW / 64) < 768) rc /= 2;
+        hipLaunchKernelGGL((k_iwt2m<NF, NT, TXW, CT, XT>), dim3(tiles, (unsigned)groups(rc)), dim3(TXW), 0, st, C, u, f.nx,
+                           f.ny, step, rc, T, alpha, beta, base, lp);
+    };
+    const size_t rows = (size_t)f.ny + (size_t)step * 64;   // bounds the launch's second dimension
+    if (4 * h <= 64 && rows / 4 <= 65535) go(std::integral_constant<int, 64>{});
+    else if (4 * h <= 256 && rows / 4 <= 65535) go(std::integral_constant<int, 256>{});
+    else
+        hipLaunchKernelGGL((k_iwt2<NF, NT, CT, XT>), dim3((unsigned)(((size_t)f.nx * f.ny + 255) / 256)), dim3(256), 0, st, C, u,
+                           f.nx, f.ny, step, T, alpha, beta, base, lp);
 }
 
 // ----------------------------------------------- fused coefficient updates --
@@ -801,9 +904,7 @@ static hipError_t iwt_t(const FlFrameDesc& f, const void* C, void* u, int level,
             }
         });
     else
-        FL_FRAME_SWITCH(f.kind, hipLaunchKernelGGL((k_iwt2<NF, NT, CT, XT>), dim3(nblk(n)), dim3(256), 0, st,
-                                                   (const CT*)C, (XT*)u, f.nx, f.ny, step, T, alpha, beta,
-                                                   base, lp));
+        FL_FRAME_SWITCH(f.kind, (launch_iwt2<NF, NT, CT, XT>)(f, (const CT*)C, (XT*)u, step, T, alpha, beta, base, lp, st));
     return hipGetLastError();
 }
 
