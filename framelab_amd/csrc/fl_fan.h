@@ -80,15 +80,6 @@ __device__ __forceinline__ float fl_fan_ray_sum(const VT* __restrict__ x, const 
 constexpr int GAO_WA = 4;
 constexpr int GAO_D = 4;
 
-// s in [1, 4]: sqrtf(s)
-__device__ __forceinline__ float fl_sqrt_one(float s)
-{
-    const float r = __builtin_amdgcn_sqrtf(s);
-    const float rd = __uint_as_float(__float_as_uint(r) - 1u), ru = __uint_as_float(__float_as_uint(r) + 1u);
-    const float lo = fmaf(-rd, r, s) <= 0.0f ? rd : r;
-    return fmaf(-ru, r, s) > 0.0f ? ru : lo;
-}
-
 // v of lane Q of this lane's quad
 template <int Q>
 __device__ __forceinline__ float fl_quad(float v)
@@ -136,7 +127,7 @@ __device__ __forceinline__ float fl_fan_gao_sum(const VT* __restrict__ x, const 
             const bool ok2 = in && !one && (unsigned)c2 < (unsigned)nv;
             const Idx col = (Idx)iu * su;
             const float xa = fl_load(x, ok1 ? col + (Idx)c1 * sv : (Idx)0), xb = fl_load(x, ok2 ? col + (Idx)c2 * sv : (Idx)0);
-            const float d = vb - va, l = fl_sqrt_one(d * d + 1.0f);
+            const float d = vb - va, l = fl_sqrt_mid(d * d + 1.0f);
             const float r0 = __builtin_amdgcn_rcpf(d), r = fmaf(fmaf(-d, r0, 1.0f), r0, r0);
             const float wa = one ? l : sid_div(fb - va, d, r) * l, wb = sid_div(vb - fb, d, r) * l;
             t1[k] = ok1 ? wa * xa : 0.0f;
