@@ -82,8 +82,8 @@ __global__ __launch_bounds__(64) void k_bfwd(const float* __restrict__ X, float*
                 const bool live = slot < f.nslots && id < f.na;
                 const int ia = min(id, f.na - 1);
                 float v;
-                if (fl_fan_small(f.nx, f.ny)) v = GAO ? fl_fan_gao_sum<true>(x, f, iv, ia) : fl_fan_ray_sum<true>(x, f, iv, ia, live);
-                else v = GAO ? fl_fan_gao_sum<false>(x, f, iv, ia) : fl_fan_ray_sum<false>(x, f, iv, ia, live);
+                if (fl_fan_small(f.nx, f.ny)) v = GAO ? fl_fan_gao_sum<true>(x, f, iv, ia) : fl_fan_ray_sum<FAN_ROWS>(x, f, iv, ia, live);
+                else v = GAO ? fl_fan_gao_sum<false>(x, f, iv, ia) : fl_fan_ray_sum<FAN_LARGE>(x, f, iv, ia, live);
                 if (live && (!GAO || (threadIdx.x & 3) == 0)) y[(size_t)slot * f.na + id] = v;
             }
         }

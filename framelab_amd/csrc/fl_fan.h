@@ -28,10 +28,14 @@ constexpr int FAN_WA = 8;
 // Image sizes whose byte offsets fit 32 bits (the tracked walk's).
 __host__ __device__ inline bool fl_fan_small(int nx, int ny) { return (size_t)nx * ny < ((size_t)1 << 30); }
 
+// How a fan ray reads its image: by 64-bit indices (the walk without tracking),
+// row by row, or a copy in bricks.
+enum FanRead { FAN_LARGE, FAN_ROWS, FAN_BRICKS };
+
 // Siddon ray sum of fan ray (view iv, cell id), scaled
 // (Ax_fan_mf_cpu_siddon.cpp:32-91): called by every lane of a wave, live = the
 // lane has a ray.
-template <bool SMALL, typename VT>
+template <int READ, typename VT>
 __device__ __forceinline__ float fl_fan_ray_sum(const VT* __restrict__ x, const FwdGeom& g, int iv, int id, bool live)
 {
     const float c = g.cs[iv], s = g.sn[iv];
@@ -41,12 +45,13 @@ __device__ __forceinline__ float fl_fan_ray_sum(const VT* __restrict__ x, const 
     const float y2 = s * g.OD + c * yd;
     const float dx = x2 - x1, dy = y2 - y1;
     const float L = sqrtf(dx * dx + dy * dy);
-    if constexpr (SMALL) {
+    if constexpr (READ != FAN_LARGE) {
+        using Layout = std::conditional_t<READ == FAN_BRICKS, FanBricks<sizeof(VT)>, FanImage<sizeof(VT)>>;
         WalkAxis ax, ay, az;
         walk_axis_init(ax, x1, dx, 1.0f, g.nx);
         walk_axis_init(ay, y1, dy, 1.0f, g.ny);
         walk_axis_init(az, 0.0f, 0.0f, 1.0f, 2);
-        return walk_rays<false, true, false>(ax, ay, az, L, live, x, FanImage<sizeof(VT)>(g.nx, g.ny)) * g.scale;
+        return walk_rays<false, true, false>(ax, ay, az, L, live, x, Layout(g.nx, g.ny)) * g.scale;
     } else {
         SidAxis ax, ay, az;
         sid_axis_init(ax, x1, dx, 1.0f, g.nx);

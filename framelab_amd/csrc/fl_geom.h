@@ -18,8 +18,8 @@ struct FwdGeom {
     // detector index maps for voxel shadows: cell a is at y_det[0] + a*pitch
     float ya0, inv_pa, zb0, inv_pb;
     int tile;               // cone forward launch shape, 0..FL_FWD_NTILES-1
-    void* bricks;           // cone: bricked copy of the input frames (plan-owned)
-    bool tracked;           // cone: it has room for the tracked walk's padded layout
+    void* bricks;           // bricked copy of the input frames (plan-owned; fan: null where there is none)
+    bool tracked;           // it has room for the tracked walk's layout
 };
 
 // One entry of a fan plan's frame -> views lists: what the pixel-driven

@@ -104,6 +104,36 @@ struct FanImage {
     __device__ __forceinline__ unsigned at(int tx, int ty, int) const { return fx(tx) + fy(ty); }
 };
 
+// Fan images in 4 x 4 bricks, brick counts along x rounded up to powers of two:
+// as ConeBricks without z.  An offset outside reads the last pixel.
+template <unsigned E>
+struct FanBricks {
+    static constexpr bool MASKED = true;
+    int lx;
+    unsigned mx, my, last;
+    static constexpr unsigned mz = ~0u;
+    __host__ __device__ FanBricks(int nx, int ny)
+    {
+        lx = 0;
+        while ((4 << lx) < nx) lx++;
+        mx = (3u | ((1u << lx) - 1) << 4) * E;
+        my = ~mx & (0u - E);
+        last = (unsigned)frame(ny) * E - E;
+    }
+    __host__ __device__ size_t frame(int ny) const { return ((size_t)16 << lx) * ((ny + 3) / 4); }
+    __device__ __forceinline__ unsigned fx(int t) const { return (((unsigned)t & 3u) | ((unsigned)t >> 2) << 4) * E & mx; }
+    __device__ __forceinline__ unsigned fy(int t) const
+    {
+        return (((unsigned)t & 3u) << 2 | ((unsigned)t >> 2) << (4 + lx)) * E & my;
+    }
+    __device__ __forceinline__ unsigned fz(int) const { return 0u; }
+    __device__ __forceinline__ unsigned stepx(int st) const { return st > 0 ? 0u - mx : 0u - E; }
+    __device__ __forceinline__ unsigned stepy(int st) const { return st > 0 ? 0u - my : 0u - E * 4; }
+    __device__ __forceinline__ unsigned stepz(int) const { return 0u; }
+    __device__ __forceinline__ unsigned place(unsigned x, unsigned y, unsigned) const { return min(x | y, last); }
+    __device__ __forceinline__ unsigned at(int tx, int ty, int) const { return fx(tx) | fy(ty); }
+};
+
 // One axis of the walk: next plane (parameter a, coordinate index p), tracked
 // cell (field f, as a byte offset, and its step), constants.
 struct WalkAxis {
@@ -150,8 +180,11 @@ __device__ __forceinline__ void walk_cross(WalkAxis& q, float an, unsigned m, ui
     float num, quo;
     if constexpr (UNIFORM && MASKED && S1) WALK_CROSS_ASM("", "%1", WALK_MASK, "s");
     else if constexpr (UNIFORM && MASKED) WALK_CROSS_ASM(WALK_SCALE, "%3", WALK_MASK, "s");
-    else {
-        static_assert(S1 && !UNIFORM && !MASKED, "a form in use");
+    else if constexpr (MASKED) {
+        static_assert(S1, "a form in use");
+        WALK_CROSS_ASM("", "%1", WALK_MASK, "v");
+    } else {
+        static_assert(S1 && !UNIFORM, "a form in use");
         WALK_CROSS_ASM("", "%1", "", "v");
     }
 }

@@ -114,6 +114,15 @@ size_t fl_tracked_frame_elems(int nx, int ny, int nz)
     return frame <= ((size_t)1 << 30) ? frame : 0;
 }
 
+// Elements of a fan image's bricked copy, 0 where its 32-bit byte offsets do not
+// reach.
+size_t fl_fan_brick_elems(int nx, int ny)
+{
+    if (nx >= (1 << 26) || ny >= (1 << 26)) return 0;
+    const size_t frame = FanBricks<4>(nx, ny).frame(ny);
+    return frame < ((size_t)1 << 30) ? frame : 0;
+}
+
 // The bricked layouts' index arithmetic needs a brick slab of under 2^24
 // elements, under 2^24 slabs and, as its in-frame offsets are 32-bit, a
 // bricked frame of at most 2^32 elements (the padding to whole bricks can
@@ -236,7 +245,20 @@ __global__ __launch_bounds__(256, 6) void k_fwd_cone_tr(const VT* __restrict__ X
     if (live) fl_store(Y, ((size_t)slot * g.nb + ib) * g.na + ia, acc * g.scale);
 }
 
-template <typename VT, typename YT, bool SMALL>
+template <typename VT>
+__global__ __launch_bounds__(256) void k_to_fan_bricks(const VT* __restrict__ x, VT* __restrict__ xb, int nx, int ny, size_t n)
+{
+    const FanBricks<sizeof(VT)> br(nx, ny);
+    const unsigned npix = (unsigned)nx * (unsigned)ny;
+    const size_t frame = br.frame(ny);
+    for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (size_t)gridDim.x * 256) {
+        const size_t f = i / npix;
+        const unsigned v = (unsigned)(i - f * npix), ty = v / (unsigned)nx, tx = v - ty * (unsigned)nx;
+        *(VT*)((char*)(xb + f * frame) + br.at((int)tx, (int)ty, 0)) = x[i];
+    }
+}
+
+template <typename VT, typename YT, int READ>
 __global__ __launch_bounds__(256) void k_fwd_fan(const VT* __restrict__ X, YT* __restrict__ Y, FwdGeom g)
 {
     constexpr int WA = FAN_WA, WV = 64 / WA;   // a wave's cells and views
@@ -246,7 +268,8 @@ __global__ __launch_bounds__(256) void k_fwd_fan(const VT* __restrict__ X, YT* _
     const int id = (int)(b % tiles) * 4 * WA + (int)(threadIdx.x >> 6) * WA + (int)threadIdx.x % WA;
     const bool live = slot < g.nslots && id < g.na;
     const int iv = g.slot_view[min(slot, g.nslots - 1)];
-    const float v = fl_fan_ray_sum<SMALL>(X + (size_t)g.view_frame[iv] * g.nvox, g, iv, min(id, g.na - 1), live);
+    const size_t frame = READ == FAN_BRICKS ? FanBricks<sizeof(VT)>(g.nx, g.ny).frame(g.ny) : g.nvox;
+    const float v = fl_fan_ray_sum<READ>(X + (size_t)g.view_frame[iv] * frame, g, iv, min(id, g.na - 1), live);
     if (live) fl_store(Y, (size_t)slot * g.na + id, v);
 }
 
@@ -349,10 +372,16 @@ static hipError_t launch_fan_t(const void* X, void* Y, const FwdGeom& g, hipStre
     const uint32_t grid = (uint32_t)((g.na + 4 * FAN_WA - 1) / (4 * FAN_WA)) *
                           (uint32_t)((g.nslots + 64 / FAN_WA - 1) / (64 / FAN_WA));
     if (grid == 0) return hipSuccess;
-    if (fl_fan_small(g.nx, g.ny))
-        hipLaunchKernelGGL((k_fwd_fan<VT, YT, true>), dim3(grid), dim3(256), 0, st, (const VT*)X, (YT*)Y, g);
-    else
-        hipLaunchKernelGGL((k_fwd_fan<VT, YT, false>), dim3(grid), dim3(256), 0, st, (const VT*)X, (YT*)Y, g);
+    if (g.tracked) {
+        const size_t n = g.nvox * (size_t)g.nframes;
+        hipLaunchKernelGGL((k_to_fan_bricks<VT>), dim3((unsigned)std::min<size_t>((n + 255) / 256, 8192)), dim3(256), 0, st,
+                           (const VT*)X, (VT*)g.bricks, g.nx, g.ny, n);
+        hipLaunchKernelGGL((k_fwd_fan<VT, YT, FAN_BRICKS>), dim3(grid), dim3(256), 0, st, (const VT*)g.bricks, (YT*)Y, g);
+    } else if (fl_fan_small(g.nx, g.ny)) {
+        hipLaunchKernelGGL((k_fwd_fan<VT, YT, FAN_ROWS>), dim3(grid), dim3(256), 0, st, (const VT*)X, (YT*)Y, g);
+    } else {
+        hipLaunchKernelGGL((k_fwd_fan<VT, YT, FAN_LARGE>), dim3(grid), dim3(256), 0, st, (const VT*)X, (YT*)Y, g);
+    }
     return hipGetLastError();
 }
 

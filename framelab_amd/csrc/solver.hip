@@ -402,10 +402,10 @@ int normal_op(fl_plan_s* pl, Workspace& w, const float* x, const void* xlo, int 
     const int kind = (flags & FL_SOLVE_MATCHED) ? FL_ADJ_MATCHED : FL_ADJ_EXACT;
     int rc;
     if (lt == FL_F32) {
-        if ((rc = fl_forward(pl, x, FL_F32, w.sino, FL_F32, st))) return rc;
+        if ((rc = fl_forward_ordered(pl, x, FL_F32, w.sino, FL_F32, st, true))) return rc;
         return fl_adjoint(pl, w.sino, FL_F32, out, FL_F32, kind, st);
     }
-    if ((rc = fl_forward(pl, xlo, lt, w.slo, lt, st))) return rc;
+    if ((rc = fl_forward_ordered(pl, xlo, lt, w.slo, lt, st, true))) return rc;
     return fl_adjoint(pl, w.slo, lt, out, FL_F32, kind, st);
 }
 
