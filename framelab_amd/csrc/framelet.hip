@@ -137,6 +137,86 @@ __global__ __launch_bounds__(256) void k_fwt3(const XT* __restrict__ u, CT* __re
     for (int b = 0; b < NF * NF * NF; b++) fl_store_nt(C, (size_t)b * nvox + idx, out[b]);
 }
 
+// Four coefficients at a multiple of four, nontemporal.
+template <typename CT>
+__device__ __forceinline__ void store4_nt(CT* p, size_t i, const float (&v)[4])
+{
+    typedef unsigned vec __attribute__((ext_vector_type(sizeof(CT))));   // 16 or 8 bytes
+    CT e[4];
+#pragma unroll
+    for (int k = 0; k < 4; k++) fl_store(e, k, v[k]);
+    vec w;
+    __builtin_memcpy(&w, e, sizeof w);
+    __builtin_nontemporal_store(w, (vec*)(p + i));
+}
+
+// k_fwt3 for three undilated taps and rows of a multiple of four voxels: four
+// neighbours in x per thread share their taps' reads and y pass, and a band's
+// store is 16 bytes a lane (FP32).  The operations of a coefficient and their
+// order are k_fwt3's.  256^3, linear FP32: 390 -> 337 us (5.6 TB/s); rows of 16
+// or 32 lanes 339 and 354.
+template <int NF, typename XT, typename CT>
+__global__ __launch_bounds__(256) void k_fwt3v(const XT* __restrict__ u, CT* __restrict__ C, int nx, int ny, int nz,
+                                              int z0, FlTaps T)
+{
+    const size_t nvox = (size_t)nx * ny * nz;
+    const int x = ((int)blockIdx.x * 64 + (int)(threadIdx.x & 63)) * 4;
+    const int y = (int)blockIdx.y * 4 + (int)(threadIdx.x >> 6);
+    const int z = z0 + (int)blockIdx.z;
+    if (x >= nx || y >= ny) return;
+    const int xl = x > 0 ? x - 1 : nx - 1, xr = x + 4 < nx ? x + 4 : 0;
+    float nb[3][3][6];
+#pragma unroll
+    for (int kz = 0; kz < 3; kz++)
+#pragma unroll
+        for (int ky = 0; ky < 3; ky++) {
+            const XT* __restrict__ row = u + ((size_t)wrap_near(z + kz - 1, nz) * ny + wrap_near(y + ky - 1, ny)) * nx;
+            nb[kz][ky][0] = fl_load(row, xl);
+#pragma unroll
+            for (int e = 0; e < 4; e++) nb[kz][ky][1 + e] = fl_load(row, x + e);
+            nb[kz][ky][5] = fl_load(row, xr);
+        }
+    const size_t idx = ((size_t)z * ny + y) * nx + x;
+#pragma unroll
+    for (int i = 0; i < NF; i++) {
+        float ty[3][6];   // corr_y with D_i
+#pragma unroll
+        for (int kz = 0; kz < 3; kz++)
+#pragma unroll
+            for (int e = 0; e < 6; e++) {
+                float s = 0.0f;
+#pragma unroll
+                for (int ky = 0; ky < 3; ky++) s = __builtin_fmaf(T.D[i][ky], nb[kz][ky][e], s);
+                ty[kz][e] = s;
+            }
+#pragma unroll
+        for (int j = 0; j < NF; j++) {
+            float tx[3][4];   // then corr_x with D_j
+#pragma unroll
+            for (int kz = 0; kz < 3; kz++)
+#pragma unroll
+                for (int e = 0; e < 4; e++) {
+                    float s = 0.0f;
+#pragma unroll
+                    for (int kx = 0; kx < 3; kx++) s = __builtin_fmaf(T.D[j][kx], ty[kz][e + kx], s);
+                    tx[kz][e] = s;
+                }
+#pragma unroll
+            for (int k = 0; k < NF; k++) {
+                float out[4];
+#pragma unroll
+                for (int e = 0; e < 4; e++) {
+                    float s = 0.0f;
+#pragma unroll
+                    for (int kz = 0; kz < 3; kz++) s = __builtin_fmaf(T.D[k][kz], tx[kz][e], s);
+                    out[e] = s;
+                }
+                store4_nt(C, (size_t)(i + NF * j + NF * NF * k) * nvox + idx, out);
+            }
+        }
+    }
+}
+
 // u = alpha * sum_b corr(R-stencil of b, C_b) + beta * base (base may be null)
 // `base` may alias `u` (out = alpha*W^T C + beta*out): each thread reads and
 // writes only its own element.
@@ -853,6 +933,13 @@ static hipError_t fwt_t(const FlFrameDesc& f, const void* u, void* C, int level,
             for (int z0 = 0; z0 < f.nz; z0 += 65535) {
                 const dim3 grid((unsigned)((f.nx + 63) / 64), (unsigned)((f.ny + 3) / 4),
                                 (unsigned)std::min(65535, f.nz - z0));
+                if constexpr (NT == 3) {
+                    if (near && step == 1 && f.nx % 4 == 0 && ((uintptr_t)u | (uintptr_t)C) % 16 == 0) {
+                        hipLaunchKernelGGL((k_fwt3v<NF, XT, CT>), dim3((unsigned)((f.nx + 255) / 256), grid.y, grid.z),
+                                           dim3(256), 0, st, (const XT*)u, (CT*)C, f.nx, f.ny, f.nz, z0, T);
+                        continue;
+                    }
+                }
                 if (near)
                     hipLaunchKernelGGL((k_fwt3<NF, NT, true, XT, CT>), grid, dim3(256), 0, st, (const XT*)u,
                                        (CT*)C, f.nx, f.ny, f.nz, z0, step, T);

@@ -1,4 +1,5 @@
-"""The marching 2D synthesis at its edges (images narrower than a tile's halo,
+"""The 3D analysis of four neighbours a thread at its edges (one to few voxels a
+side, rows around a workgroup's), the marching 2D synthesis at its edges (images narrower than a tile's halo,
 widths and heights around a tile's and a run's, every tile form up to the
 gather, dilations larger than the image) and the soft threshold at block
 edges, odd band sizes and each storage type."""
@@ -48,3 +49,19 @@ def test_soft_threshold(gpu, shape, dtype):
     dim = 3 if shape[1] == 27 else 2
     got = FrameletExpansion(dim, FrameletSystem(dim, kind, shape[0]), a).softThreshold(0.25).frameletArray
     assert torch.equal(got, want)
+
+
+@pytest.mark.parametrize("kind", ["haar", "linear"])
+@pytest.mark.parametrize("shape", [(1, 1, 4), (2, 2, 4), (3, 5, 8), (4, 4, 256), (2, 3, 260), (2, 9, 12), (3, 4, 10)])
+def test_analysis3(gpu, oracle, shape, kind):
+    from framelab_amd.framelets import FrameletSystem
+    u = np.random.default_rng(shape[2]).standard_normal(shape).astype(np.float32)
+    W = FrameletSystem(3, kind, 1)
+    x = torch.from_numpy(u).to(gpu)
+    c = W.forwardTransform(x).frameletArray
+    D, _ = oracle.framelet_filters(kind)
+    nf = len(D)
+    ref = oracle.fradec3d(u.astype(np.float64), D, 1)[0]
+    want = np.stack([ref[i, j, k] for k in range(nf) for j in range(nf) for i in range(nf)])
+    assert _rel(c[0].cpu().numpy(), want) < 2e-6
+    assert torch.equal(W.forwardTransform(x, coef_dtype=torch.bfloat16).frameletArray, c.to(torch.bfloat16))
