@@ -412,27 +412,31 @@ LT* lowp_copy(Workspace& w)
     return std::is_same<LT, float>::value ? nullptr : (LT*)w.plo;
 }
 
-// q = A^T (A x) for x the FP32 vector (or its low-precision copy)
-int normal_op(fl_plan_s* pl, Workspace& w, const float* x, const void* xlo, int flags, float* out, hipStream_t st)
+// q = A^T (A x) for x the FP32 vector (or its low-precision copy).  `captured`:
+// cg_run records it into its own graph, whose replays it orders against the
+// plan's other forwards; a capture that a caller began is replayed in no such
+// order, so its forwards must not use the plan's bricks (fl_forward_ordered).
+int normal_op(fl_plan_s* pl, Workspace& w, const float* x, const void* xlo, int flags, float* out, hipStream_t st,
+              bool captured)
 {
     const int lt = lowp_type(flags);
     const int kind = (flags & FL_SOLVE_MATCHED) ? FL_ADJ_MATCHED : FL_ADJ_EXACT;
     int rc;
     if (lt == FL_F32) {
-        if ((rc = fl_forward_ordered(pl, x, FL_F32, w.sino, FL_F32, st, true))) return rc;
+        if ((rc = fl_forward_ordered(pl, x, FL_F32, w.sino, FL_F32, st, captured))) return rc;
         return fl_adjoint(pl, w.sino, FL_F32, out, FL_F32, kind, st);
     }
-    if ((rc = fl_forward_ordered(pl, xlo, lt, w.slo, lt, st, true))) return rc;
+    if ((rc = fl_forward_ordered(pl, xlo, lt, w.slo, lt, st, captured))) return rc;
     return fl_adjoint(pl, w.slo, lt, out, FL_F32, kind, st);
 }
 
 template <typename LT>
-int cg_body_t(fl_plan_s* pl, Workspace& w, float* u, float lam, int flags, hipStream_t st)
+int cg_body_t(fl_plan_s* pl, Workspace& w, float* u, float lam, int flags, hipStream_t st, bool captured)
 {
     const size_t n = (size_t)pl->nvox * pl->nt;
     const unsigned g = grid_for(n);
     int rc;
-    if ((rc = normal_op(pl, w, w.p, w.plo, flags, w.q, st))) return rc;
+    if ((rc = normal_op(pl, w, w.p, w.plo, flags, w.q, st, captured))) return rc;
     hipLaunchKernelGGL(k_cg_pq, dim3(g), dim3(256), 0, st, w.q, w.p, lam, n, w.part, w.st);
     hipLaunchKernelGGL(k_cg_update, dim3(g), dim3(256), 0, st, u, w.r, w.p, w.q, n, w.part, w.part_r, w.st);
     hipLaunchKernelGGL((k_cg_p<LT>), dim3(g), dim3(256), 0, st, w.p, w.r, lowp_copy<LT>(w), n, w.part_r, w.st, w.log,
@@ -441,12 +445,12 @@ int cg_body_t(fl_plan_s* pl, Workspace& w, float* u, float lam, int flags, hipSt
     return FL_OK;
 }
 
-int cg_body(fl_plan_s* pl, Workspace& w, float* u, float lam, int flags, hipStream_t st)
+int cg_body(fl_plan_s* pl, Workspace& w, float* u, float lam, int flags, hipStream_t st, bool captured)
 {
     switch (lowp_type(flags)) {
-    case FL_BF16: return cg_body_t<bf16_t>(pl, w, u, lam, flags, st);
-    case FL_F16: return cg_body_t<f16_t>(pl, w, u, lam, flags, st);
-    default: return cg_body_t<float>(pl, w, u, lam, flags, st);
+    case FL_BF16: return cg_body_t<bf16_t>(pl, w, u, lam, flags, st, captured);
+    case FL_F16: return cg_body_t<f16_t>(pl, w, u, lam, flags, st, captured);
+    default: return cg_body_t<float>(pl, w, u, lam, flags, st, captured);
     }
 }
 
@@ -459,10 +463,10 @@ int cg_init_t(fl_plan_s* pl, Workspace& w, const float* b, float* u, float lam, 
     hipLaunchKernelGGL(k_state_init, dim3(1), dim3(1), 0, st, w.st, tol);
     int rc;
     if (lowp_type(flags) == FL_F32) {
-        rc = normal_op(pl, w, u, nullptr, flags, w.q, st);
+        rc = normal_op(pl, w, u, nullptr, flags, w.q, st, false);
     } else {
         hipLaunchKernelGGL((k_cast<LT>), dim3(g), dim3(256), 0, st, u, lowp_copy<LT>(w), n);
-        rc = normal_op(pl, w, nullptr, w.plo, flags, w.q, st);
+        rc = normal_op(pl, w, nullptr, w.plo, flags, w.q, st, false);
     }
     if (rc) return rc;
     hipLaunchKernelGGL((k_cg_init<LT>), dim3(g), dim3(256), 0, st, w.q, u, b, lam, w.r, w.p, lowp_copy<LT>(w), n,
@@ -499,7 +503,7 @@ int cg_run(fl_plan_s* pl, Workspace& w, const float* b, float* u_caller, float l
         if (!hit) {
             drop_graph(w);
             HIPCHK(hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal));
-            rc = cg_body(pl, w, u, lam, flags, st);
+            rc = cg_body(pl, w, u, lam, flags, st, true);
             hipGraph_t gr = nullptr;
             hipError_t e = hipStreamEndCapture(st, &gr);
             if (rc) {
@@ -525,7 +529,7 @@ int cg_run(fl_plan_s* pl, Workspace& w, const float* b, float* u_caller, float l
         }
     } else {
         for (int k = 0; k < iters; k++)
-            if ((rc = cg_body(pl, w, u, lam, flags, st))) return rc;
+            if ((rc = cg_body(pl, w, u, lam, flags, st, false))) return rc;
     }
     HIPCHK(fl_launch_copy(u, u_caller, n, st));
     return FL_OK;
