@@ -430,6 +430,14 @@ extern "C" int fl_plan_create(fl_plan* out, const fl_geometry* g)
         f.inv_pa = a.inv_pa = (float)(1.0 / pa);
         f.zb0 = a.zb0 = cone ? g->z_det[0] : 0.0f;
         f.inv_pb = a.inv_pb = (float)(1.0 / pb);
+        // (a panel 2^40 voxels away has no precision left to lose)
+        double y2 = 0.0, z2 = 0.0;
+        for (int k = 0; k < g->na; k++) y2 = fmax(y2, (double)g->y_det[k] * g->y_det[k]);
+        for (int k = 0; cone && k < g->nb; k++) z2 = fmax(z2, (double)g->z_det[k] * g->z_det[k]);
+        const double SD = (double)g->SO + g->OD, len = sqrt(SD * SD + y2 + z2);
+        const int e = len < 0x1p40 ? std::max(ilogb(len) + 1, 0) : 0;
+        f.seg_up = ldexpf(1.0f, e);
+        f.seg_down = ldexpf(1.0f, -e);
         // deviation from the uniform grids the window maps assume
         double dev = 0.0;
         for (int k = 0; k < g->na && pa != 0.0; k++)

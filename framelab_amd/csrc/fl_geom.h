@@ -17,6 +17,8 @@ struct FwdGeom {
     size_t nvox;            // voxels per frame
     // detector index maps for voxel shadows: cell a is at y_det[0] + a*pitch
     float ya0, inv_pa, zb0, inv_pb;
+    // cone: 2^e above every ray's length, and 2^-e (the matched adjoint's scaling)
+    float seg_up, seg_down;
     int tile;               // cone forward launch shape, 0..FL_FWD_NTILES-1
     void* bricks;           // bricked copy of the input frames (plan-owned; fan: null where there is none)
     bool tracked;           // it has room for the tracked walk's layout

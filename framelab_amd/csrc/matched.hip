@@ -79,6 +79,12 @@ struct MatchedLds {
 // along z, so the test is on the differences that involve z planes, and a
 // column whose own interval is that short sends its rows there outright.
 //
+// The staged directions are 2^-e times the forward's, 2^e above every |d|
+// (FwdGeom::seg_up): |d| times a value near the type's largest would overflow
+// where the term does not.  Plane parameters, segments and tau are 2^e times
+// the forward's for it, exactly, and the factors cancel in a midpoint's
+// coordinates and in a term.
+//
 // VG groups share a brick's views between them and add their sums in group
 // order.
 //
@@ -124,7 +130,7 @@ __global__ __launch_bounds__(256 * VG, 4) void k_adj_matched_cone(
     constexpr bool dz_one = DZ1;
     // tau's constants (fl_walk.h): plane parameters reach at most A here
     const float rc = 0.5f * sqrtf((float)f.nx * f.nx + (float)f.ny * f.ny);
-    const float A4 = 4.0f * 1.01f * (f.SO + rc + 1.0f) / SD;
+    const float A4 = 4.0f * 1.01f * (f.SO + rc + 1.0f) / SD * f.seg_up;
     const float wx = 1.5f * (float)f.nx + 3.0f, wy = 1.5f * (float)f.ny + 3.0f;
     const float wz = DZ1 ? 1.5f * (float)f.nz + 3.0f : f.dz0 * (2.5f * (float)f.nz + 5.0f);
     float acc[KZ];
@@ -196,7 +202,7 @@ __global__ __launch_bounds__(256 * VG, 4) void k_adj_matched_cone(
         if (v.fits) {
             if (wv == 0 && lane < v.nA) {
                 const float x1 = v.c * (-f.SO), y1 = v.s * (-f.SO), yd = f.ydet[v.A0 + lane];
-                const float dx = (v.c * f.OD - v.s * yd) - x1, dy = (v.s * f.OD + v.c * yd) - y1;
+                const float dx = ((v.c * f.OD - v.s * yd) - x1) * f.seg_down, dy = ((v.s * f.OD + v.c * yd) - y1) * f.seg_down;
                 const float rx = 1.0f / dx, ry = 1.0f / dy;
                 t.dx[p][lane] = dx;
                 t.dy[p][lane] = dy;
@@ -206,7 +212,7 @@ __global__ __launch_bounds__(256 * VG, 4) void k_adj_matched_cone(
                 t.tc[p][lane] = 1.01f * 0x1p-23f * (A4 + fmaxf(wx * fabsf(rx), wy * fabsf(ry)));
             }
             if (wv == 1 && lane < v.nB) {
-                const float dz = (f.zdet[v.B0 + lane] + v.sz) - v.sz;
+                const float dz = ((f.zdet[v.B0 + lane] + v.sz) - v.sz) * f.seg_down;
                 const float rz = 1.0f / dz;
                 t.dz[p][lane] = dz;
                 t.rz[p][lane] = rz;

@@ -93,3 +93,22 @@ def test_values_stay_with_their_rays(gpu):
     x = P.adjoint(Y, kind=ADJ_MATCHED)
     bad = ~torch.isfinite(x)
     assert bad.any() and bad.sum() <= 24 * 27
+
+
+# tables of each launch form; a power of two scales every operation exactly
+@pytest.mark.parametrize("case", [CASES[1], CASES[5], CASES[8], CASES[10]])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_large_values(gpu, case, dtype):
+    """Values up to 2^123 (1e37): nothing overflows that the sums do not."""
+    from framelab_amd.projector import ADJ_MATCHED, Projector
+    p = _para(case)
+    P = Projector(p)
+    Y = torch.from_numpy(np.random.default_rng(5).uniform(-1, 1, P.sino_shape).astype(np.float32)).to(gpu).to(dtype)
+    k = 119 if p.nv > 8 else 123   # voxel sums of so many views of up to 2 |y| stay finite
+    x = P.adjoint(Y, kind=ADJ_MATCHED, dtype=torch.float32)
+    assert torch.equal(P.adjoint(Y * 2.0 ** k, kind=ADJ_MATCHED, dtype=torch.float32), x * 2.0 ** k)
+
+
+def test_columns_down(gpu):
+    p = _para((26, 22, 36, 33, 41, 20, 1.0, 3.0))
+    _check(gpu, dataclasses.replace(p, y_det=p.y_det[::-1].copy()))
