@@ -55,7 +55,7 @@ template <int KZ>
 struct ExactLds {
     static constexpr int N = KZ == 8 ? 1152 : 1408;   // footprint cells (four workgroups' tables fit a CU)
     float2 zs[N], xs[N];
-    float y[N];
+    float y[N + 1];       // (and a zero)
     float acc[KZ][256];   // the voxels' sums (a rolled loop over k indexes them)
     float a[2][FP_A], b[2][FP_A], ra[2][FP_A], rb[2][FP_A], sba[2][FP_A], sab[2][FP_A];
     float c[2][FP_B], rc[2][FP_B], ch[2][FP_B];   // (ch: a slice's half height signed by c)
@@ -129,6 +129,7 @@ __global__ __launch_bounds__(256, 4) void k_adj_cone_zc(const YT* __restrict__ Y
     const float tz = 1.5f * fmaxf(fabsf(g.zdet[0]), fabsf(g.zdet[nb - 1])) / SD;
 #pragma unroll
     for (int k = 0; k < KZ; k++) t.acc[k][tid] = 0.0f;
+    if (tid == 0) t.y[t.N] = 0.0f;
 
     // 64 views at a time are set up one per lane: source and direction,
     // sinogram slot and the brick's footprint on the panel
@@ -343,9 +344,12 @@ __global__ __launch_bounds__(256, 4) void k_adj_cone_zc(const YT* __restrict__ Y
             constexpr int CA = decltype(ca)::value;
             // per column: (x, y) of the ray's entry into and exit from the
             // square, the chord's share, and per end the slope of z on its face
-            // (place in zs) and the face's distance from the source and half side
+            // (place in zs) and the face's distance from the source and half side;
+            // ky + kb * ny is the value's place in y, for a lane without the column
+            // that of the zero (the shadow's last value again would make NaN of
+            // an infinite sum: 0 * inf)
             float xi[CA], yi[CA], xo[CA], yo[CA], uv[CA], ni[CA], hi[CA], no[CA], ho[CA];
-            int fi[CA], fo[CA];
+            int fi[CA], fo[CA], ny[CA], ky[CA];
             uint64_t hit[CA], full[CA];   // lanes whose ray crosses the square; that take the whole routine
             float ec = 0.0f;
 #pragma unroll
@@ -371,6 +375,8 @@ __global__ __launch_bounds__(256, 4) void k_adj_cone_zc(const YT* __restrict__ Y
                 uv[c] = du * du + dv * dv;
                 ni[c] = bex ? -p0x : -p0y; hi[c] = bex ? hx : hy;
                 no[c] = bxx ? -p0x : -p0y; ho[c] = bxx ? hx : hy;
+                ny[c] = alo + c <= ahi ? u.nA : 0;
+                ky[c] = alo + c <= ahi ? ka : t.N;
                 fi[c] = 2 * ka + (bex ? 0 : 1);
                 fo[c] = 2 * ka + (bxx ? 0 : 1);
             }
@@ -389,7 +395,7 @@ __global__ __launch_bounds__(256, 4) void k_adj_cone_zc(const YT* __restrict__ Y
                     for (int c = 0; c < CA; c++) {
                         si[c] = zs[2 * row + fi[c]];
                         so[c] = zs[2 * row + fo[c]];
-                        y[c] = t.y[row + min(alo + c, ahi)];
+                        y[c] = t.y[c == 0 ? row + alo : __mul24(kb, ny[c]) + ky[c]];
                     }
                     uint64_t odd[CA], any = 0;
                     const float hzs = t.ch[p0][kb];

@@ -74,3 +74,17 @@ def test_geometries(gpu, oracle, kind):
         phi = (np.arange(16) // 2 * (np.pi / 4) + np.where(np.arange(16) % 2, 3e-5, -2e-7)).astype(np.float32)
         p = _para(case, sd_phi=phi)
     _check(gpu, oracle, p)
+
+
+@pytest.mark.parametrize("cells", [(33, 29), (60, 44), (90, 70)])
+def test_infinite_values_count_once(gpu, cells):
+    """Infinite values far enough apart that a voxel's shadow holds one of them:
+    its sum is infinite where that cell's chord is positive, never NaN."""
+    from framelab_amd.projector import ADJ_EXACT, Projector
+    P = Projector(_para((24, 24, 24, *cells, 3, 1.0, 4.0)))
+    for a in range(0, 10, 3):
+        ones = torch.zeros(P.sino_shape, device=gpu)
+        ones[1, a::10, a::10] = 1.0
+        chord = P.adjoint(ones, kind=ADJ_EXACT)
+        x = P.adjoint(torch.where(ones > 0, torch.inf, 0.0), kind=ADJ_EXACT)
+        assert (chord > 0).any() and torch.isposinf(x[chord > 0]).all()
