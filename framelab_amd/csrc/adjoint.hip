@@ -53,9 +53,10 @@ static_assert(FP_A <= 64 && FP_B <= 64, "footprint columns / rows are staged by 
 // ahead.
 template <int KZ>
 struct ExactLds {
-    static constexpr int N = KZ == 8 ? 1152 : 1408;   // footprint cells (four workgroups' tables fit a CU)
+    static constexpr int CELLS = KZ == 8 ? 1152 : 1408;   // footprint cells (four workgroups' tables fit a CU)
+    static constexpr int N = CELLS + FP_B;                // and a zero at each row's end
     float2 zs[N], xs[N];
-    float y[N + 1];       // (and a zero)
+    float y[N];
     float acc[KZ][256];   // the voxels' sums (a rolled loop over k indexes them)
     float a[2][FP_A], b[2][FP_A], ra[2][FP_A], rb[2][FP_A], sba[2][FP_A], sab[2][FP_A];
     float c[2][FP_B], rc[2][FP_B], ch[2][FP_B];   // (ch: a slice's half height signed by c)
@@ -129,7 +130,6 @@ __global__ __launch_bounds__(256, 4) void k_adj_cone_zc(const YT* __restrict__ Y
     const float tz = 1.5f * fmaxf(fabsf(g.zdet[0]), fabsf(g.zdet[nb - 1])) / SD;
 #pragma unroll
     for (int k = 0; k < KZ; k++) t.acc[k][tid] = 0.0f;
-    if (tid == 0) t.y[t.N] = 0.0f;
 
     // 64 views at a time are set up one per lane: source and direction,
     // sinogram slot and the brick's footprint on the panel
@@ -182,7 +182,7 @@ __global__ __launch_bounds__(256, 4) void k_adj_cone_zc(const YT* __restrict__ Y
         v.nB = __builtin_amdgcn_readlane(ubn, l);
         v.off = (size_t)__builtin_amdgcn_readlane(uslot, l) * g.nd;
         v.any = v.nA > 0 && v.nB > 0;
-        v.fits = v.nA <= FP_A && v.nB <= FP_B && v.nA * v.nB <= t.N;
+        v.fits = v.nA <= FP_A && v.nB <= FP_B && v.nA * v.nB <= t.CELLS;
         return v;
     };
     // a view ahead: direction components and reciprocals of the columns (wave
@@ -252,7 +252,9 @@ __global__ __launch_bounds__(256, 4) void k_adj_cone_zc(const YT* __restrict__ Y
             // the ratios' IEEE quotients from the staged reciprocals
             const uint32_t mA = fl_small_div_m((uint32_t)v.nA);
             const int cells = v.nA * v.nB;
-            auto put = [&](int k, int ka, int kb, float yk) {
+            if (tid < v.nB) t.y[__mul24(tid, v.nA + 1) + v.nA] = 0.0f;
+            auto put = [&](int i, int ka, int kb, float yk) {
+                const int k = i + kb;
                 const float a = t.a[p][ka], bb = t.b[p][ka], cc = t.c[p][kb], rc = t.rc[p][kb];
                 t.zs[k] = make_float2(fl_div_r(cc, a, t.ra[p][ka]), fl_div_r(cc, bb, t.rb[p][ka]));
                 t.xs[k] = make_float2(fl_div_r(a, cc, rc), fl_div_r(bb, cc, rc));
@@ -308,7 +310,7 @@ __global__ __launch_bounds__(256, 4) void k_adj_cone_zc(const YT* __restrict__ Y
                 return fl_chord_box3(x1, y1, z1, u.c * g.OD - u.s * yd, u.s * g.OD + u.c * yd, g.zdet[u.B0 + kb] + u.sz, 1.0f,
                                      1.0f, g.dz, xc, yc, zc);
             }
-            const float2 zs = t.zs[__mul24(kb, u.nA) + ka], xs = t.xs[__mul24(kb, u.nA) + ka];
+            const float2 zs = t.zs[__mul24(kb, u.nA + 1) + ka], xs = t.xs[__mul24(kb, u.nA + 1) + ka];
             const float h[3] = {0.5f, 0.5f, hz}, pt[3] = {p0x, p0y, z1 - zc};
             FlRatiosS q;
             q.r.sba = t.sba[p0][ka]; q.r.sab = t.sab[p0][ka];
@@ -345,11 +347,11 @@ __global__ __launch_bounds__(256, 4) void k_adj_cone_zc(const YT* __restrict__ Y
             // per column: (x, y) of the ray's entry into and exit from the
             // square, the chord's share, and per end the slope of z on its face
             // (place in zs) and the face's distance from the source and half side;
-            // ky + kb * ny is the value's place in y, for a lane without the column
-            // that of the zero (the shadow's last value again would make NaN of
-            // an infinite sum: 0 * inf)
+            // ky, the value's place in its row, is that of the zero for a lane without
+            // the column (the lane's last value again would make NaN of an
+            // infinite sum: 0 * inf)
             float xi[CA], yi[CA], xo[CA], yo[CA], uv[CA], ni[CA], hi[CA], no[CA], ho[CA];
-            int fi[CA], fo[CA], ny[CA], ky[CA];
+            int fi[CA], fo[CA], ky[CA];
             uint64_t hit[CA], full[CA];   // lanes whose ray crosses the square; that take the whole routine
             float ec = 0.0f;
 #pragma unroll
@@ -375,8 +377,7 @@ __global__ __launch_bounds__(256, 4) void k_adj_cone_zc(const YT* __restrict__ Y
                 uv[c] = du * du + dv * dv;
                 ni[c] = bex ? -p0x : -p0y; hi[c] = bex ? hx : hy;
                 no[c] = bxx ? -p0x : -p0y; ho[c] = bxx ? hx : hy;
-                ny[c] = alo + c <= ahi ? u.nA : 0;
-                ky[c] = alo + c <= ahi ? ka : t.N;
+                ky[c] = alo + c <= ahi ? ka : u.nA;
                 fi[c] = 2 * ka + (bex ? 0 : 1);
                 fo[c] = 2 * ka + (bxx ? 0 : 1);
             }
@@ -389,13 +390,13 @@ __global__ __launch_bounds__(256, 4) void k_adj_cone_zc(const YT* __restrict__ Y
                 int blo, bhi;
                 rows(zc, blo, bhi);
                 for (int kb = blo; kb <= bhi; kb++) {
-                    const int row = __mul24(kb, u.nA);
+                    const int row = __mul24(kb, u.nA + 1);
                     float si[CA], so[CA], y[CA], l[CA];
 #pragma unroll
                     for (int c = 0; c < CA; c++) {
                         si[c] = zs[2 * row + fi[c]];
                         so[c] = zs[2 * row + fo[c]];
-                        y[c] = t.y[c == 0 ? row + alo : __mul24(kb, ny[c]) + ky[c]];
+                        y[c] = t.y[row + ky[c]];
                     }
                     uint64_t odd[CA], any = 0;
                     const float hzs = t.ch[p0][kb];
@@ -409,7 +410,7 @@ __global__ __launch_bounds__(256, 4) void k_adj_cone_zc(const YT* __restrict__ Y
                         uint64_t some = hit[c] & in & out;
                         if (cross) {   // one end on a z face
                             const bool low = lanes(in);
-                            const float2 xs = t.xs[row + min(alo + c, ahi)];
+                            const float2 xs = t.xs[row + ky[c]];
                             const float hs = low ? hzs : -hzs;
                             const float pu = (xs.x * (-p2) + p0x) + xs.x * hs, pv = (xs.y * (-p2) + p0y) + xs.y * hs;
                             const float du = pu - (low ? xi[c] : xo[c]), dv = pv - (low ? yi[c] : yo[c]);
@@ -442,7 +443,7 @@ __global__ __launch_bounds__(256, 4) void k_adj_cone_zc(const YT* __restrict__ Y
                 int blo, bhi;
                 rows(zc, blo, bhi);
                 for (int kb = blo; kb <= bhi; kb++)
-                    for (int ka = alo; ka <= ahi; ka++) a = a + chord(ka, kb, zc) * t.y[__mul24(kb, u.nA) + ka];
+                    for (int ka = alo; ka <= ahi; ka++) a = a + chord(ka, kb, zc) * t.y[__mul24(kb, u.nA + 1) + ka];
                 t.acc[k][tid] = a;
             }
         }
