@@ -74,7 +74,7 @@ struct ExactLds {
 //
 // What find_l_3d tests on a box's x and y faces splits into a test along the
 // other of x and y, which depends on the detector column only, and one along
-// z.  A thread works out the former once per view for its two or three
+// z.  A thread works out the former once per view for its one to three
 // columns: usually the ray enters the (x, y) square through one face and
 // leaves through one, both known with the chord's x and y part.  A cell is
 // then the heights zi, zo at which the ray crosses those faces: both inside
@@ -93,7 +93,8 @@ struct ExactLds {
 //     or more in x or y meets no face; one that does not, and has not exactly
 //     one entry and one exit, takes the routine for all its cells, and so does
 //     one within 1/4096 of an axis's direction.
-// Shadows of more than three columns take the routine throughout.
+// The waves' usual counts of columns, CA0 and one more, have a loop of their own;
+// wider shadows take the routine throughout.
 //
 // Bound by VALU issue (some 300 instructions a voxel and view at 256^3: 1.8 rows
 // of 2.3 columns at 26, and 22 more for each that some lane leaves through a z
@@ -102,7 +103,7 @@ struct ExactLds {
 // (32 rows overflowed); 64^3, 60 views: 572 -> 299 us (before: every cell's six
 // candidates, some 90 instructions).  Four waves per SIMD; three take 55.8 ms,
 // five spill (69).
-template <typename YT, typename XT, int KZ>
+template <typename YT, typename XT, int KZ, int CA0>
 __global__ __launch_bounds__(256, 4) void k_adj_cone_zc(const YT* __restrict__ Y, XT* __restrict__ X, AdjGeom g)
 {
     constexpr int BZ = 4 * KZ;
@@ -433,8 +434,9 @@ __global__ __launch_bounds__(256, 4) void k_adj_cone_zc(const YT* __restrict__ Y
                 t.acc[k][tid] = a;
             }
         };
-        if (__builtin_amdgcn_ballot_w64(alo + 1 < ahi) == 0) slices(std::integral_constant<int, 2>{});
-        else if (__builtin_amdgcn_ballot_w64(alo + 2 < ahi) == 0) slices(std::integral_constant<int, 3>{});
+        auto most = [&](int n) { return __builtin_amdgcn_ballot_w64(alo + n <= ahi) == 0; };   // columns of a lane
+        if (most(CA0)) slices(std::integral_constant<int, CA0>{});
+        else if (most(CA0 + 1)) slices(std::integral_constant<int, CA0 + 1>{});
         else {
 #pragma unroll 1
             for (int k = 0; k < kn; k++) {
@@ -531,9 +533,20 @@ static hipError_t launch_adj_cone_t(const void* Y, void* X, const AdjGeom& g, hi
 {
     const auto blocks = [&](int kz) { return (uint32_t)((g.nx + 7) / 8) * ((g.ny + 7) / 8) * ((g.nz + 4 * kz - 1) / (4 * kz)); };
     if (blocks(4) == 0 || g.nt == 0) return hipSuccess;
+    auto launch = [&](auto kz, auto ca0) {
+        constexpr int KZ = decltype(kz)::value, CA0 = decltype(ca0)::value;
+        hipLaunchKernelGGL((k_adj_cone_zc<YT, XT, KZ, CA0>), dim3(blocks(KZ), g.nt), dim3(256), 0, st, (const YT*)Y, (XT*)X, g);
+    };
+    // Panels of under 0.9 cells a voxel (at the axis): lanes have one column or
+    // two.  N^3 voxels, one and two columns against two and three, us: 128^3, 60
+    // views, 0.33 cells 465 and 620, 0.66 604 and 695, 0.79 714 and 770, 0.99 891
+    // and 870; 256^3, 30 views, 0.33 1293 and 1714, 0.79 2085 and 2224, 0.99 2784 and
+    // 2721; 64^3, 60 views, 0.33 144 and 186, 0.99 232 and 232.  (In one kernel the
+    // three forms cost the fine panels 1.3%.)
+    const bool coarse = (g.SO + g.OD) / g.SO * fabsf(g.inv_pa) < 0.9f;
     auto go = [&](auto kz) {
-        constexpr int KZ = decltype(kz)::value;
-        hipLaunchKernelGGL((k_adj_cone_zc<YT, XT, KZ>), dim3(blocks(KZ), g.nt), dim3(256), 0, st, (const YT*)Y, (XT*)X, g);
+        if (coarse) launch(kz, std::integral_constant<int, 1>{});
+        else launch(kz, std::integral_constant<int, 2>{});
     };
     // Slices a thread: eight share a column's work best, but leave few bricks of
     // unequal cost.  N^3 voxels, 96 views, us (eight, four, two): 72^3 1486, 791,

@@ -88,3 +88,21 @@ def test_infinite_values_count_once(gpu, cells):
         chord = P.adjoint(ones, kind=ADJ_EXACT)
         x = P.adjoint(torch.where(ones > 0, torch.inf, 0.0), kind=ADJ_EXACT)
         assert (chord > 0).any() and torch.isposinf(x[chord > 0]).all()
+
+
+@pytest.mark.parametrize("case", [(24, 24, 24, 8, 7, 9, 1.0, 4.0), (40, 36, 70, 14, 60, 5, 1.0, 3.0), (34, 30, 20, 22, 5, 8, 0.5, 2.0)])
+def test_cells_wider_than_shadows(gpu, oracle, case):
+    _check(gpu, oracle, _para(case))
+
+
+@pytest.mark.parametrize("cells, columns", [((8, 7), 1), ((49, 65), 2)])
+def test_columns_by_panel(gpu, cells, columns):
+    """Panels of less than a cell a voxel take the form for one column or two."""
+    from framelab_amd import _lib
+    from framelab_amd.projector import ADJ_EXACT, Projector
+    from graph_kernels import captured_kernels
+    P = Projector(_para((24, 24, 24, *cells, 3, 1.0, 4.0)))
+    y, x = torch.zeros(P.sino_shape, device=gpu), torch.zeros(P.vol_shape, device=gpu)
+    names = captured_kernels(lambda st: _lib.check(_lib.lib().fl_adjoint(P.handle, y.data_ptr(), _lib.FL_F32, x.data_ptr(),
+                                                                         _lib.FL_F32, ADJ_EXACT, st)))
+    assert len(names) == 1 and f"k_adj_cone_zcIffLi2ELi{columns}E" in names[0]
