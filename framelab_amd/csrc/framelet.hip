@@ -137,16 +137,28 @@ __global__ __launch_bounds__(256) void k_fwt3(const XT* __restrict__ u, CT* __re
     for (int b = 0; b < NF * NF * NF; b++) fl_store_nt(C, (size_t)b * nvox + idx, out[b]);
 }
 
-// Four coefficients at a multiple of four, nontemporal.
+// a * b[k] + c[k], four coefficients at a multiple of four, nontemporal.  FP16
+// rounds product, sum and conversion once, as one such coefficient is compiled
+// in k_fwt3; of four the compiler converts some in a second rounding.
 template <typename CT>
-__device__ __forceinline__ void store4_nt(CT* p, size_t i, const float (&v)[4])
+__device__ __forceinline__ void store4_nt(CT* p, size_t i, float a, const float (&b)[4], const float (&c)[4])
 {
     typedef unsigned vec __attribute__((ext_vector_type(sizeof(CT))));   // 16 or 8 bytes
-    CT e[4];
-#pragma unroll
-    for (int k = 0; k < 4; k++) fl_store(e, k, v[k]);
     vec w;
-    __builtin_memcpy(&w, e, sizeof w);
+    if constexpr (std::is_same<CT, f16_t>::value) {
+#pragma unroll
+        for (int k = 0; k < 4; k += 2) {
+            unsigned h = 0;
+            asm("v_fma_mixlo_f16 %0, %1, %2, %3" : "+v"(h) : "s"(a), "v"(b[k]), "v"(c[k]));
+            asm("v_fma_mixhi_f16 %0, %1, %2, %3" : "+v"(h) : "s"(a), "v"(b[k + 1]), "v"(c[k + 1]));
+            w[k / 2] = h;
+        }
+    } else {
+        CT e[4];
+#pragma unroll
+        for (int k = 0; k < 4; k++) fl_store(e, k, __builtin_fmaf(a, b[k], c[k]));
+        __builtin_memcpy(&w, e, sizeof w);
+    }
     __builtin_nontemporal_store(w, (vec*)(p + i));
 }
 
@@ -203,15 +215,14 @@ __global__ __launch_bounds__(256) void k_fwt3v(const XT* __restrict__ u, CT* __r
                 }
 #pragma unroll
             for (int k = 0; k < NF; k++) {
-                float out[4];
+                float s[4];
 #pragma unroll
                 for (int e = 0; e < 4; e++) {
-                    float s = 0.0f;
+                    s[e] = 0.0f;
 #pragma unroll
-                    for (int kz = 0; kz < 3; kz++) s = __builtin_fmaf(T.D[k][kz], tx[kz][e], s);
-                    out[e] = s;
+                    for (int kz = 0; kz < 2; kz++) s[e] = __builtin_fmaf(T.D[k][kz], tx[kz][e], s[e]);
                 }
-                store4_nt(C, (size_t)(i + NF * j + NF * NF * k) * nvox + idx, out);
+                store4_nt(C, (size_t)(i + NF * j + NF * NF * k) * nvox + idx, T.D[k][2], tx[2], s);
             }
         }
     }
