@@ -930,6 +930,32 @@ static unsigned nblk(size_t n) { return (unsigned)((n + 255) / 256); }
         else { constexpr int NF = 5, NT = 5; CALL; }                                  \
     } while (0)
 
+// Whether k_fwt3v serves a volume (rows of a multiple of four).  Its waves span 256
+// voxels of a row where k_fwt3's span 64, so what counts is how many of the
+// lanes work: the share, k_fwt3's waves a row over four times its own, here in
+// eighths.  Times of k_fwt3 over those of k_fwt3v:
+//  - rows of no whole 64-byte lines, whose bands k_fwt3 writes in pieces of
+//    lines, FP32 linear: 68 x 96 x 96 1.95, 132 x 48 x 48 1.9, 264 x 96 x 96 1.40; under a
+//    share of 4, 36 x 96 x 96 0.57; under 16 MB (BF16), 116 x 48 x 48 0.96; 16-bit
+//    Haar (16 bytes a voxel) from a share of 6 on, 196 x 96 x 96 1.46, 264 x 96 x 96 0.89;
+//  - whole lines, FP32 linear: 224 x 128 x 128 1.03, 208 x 160 x 160 1.16, 448 x 200 x 200 1.04,
+//    208 x 96 x 96 0.93; a share of 6, 192 x 256 x 256 0.96, 64 x 192 x 192 0.45.  Where the
+//    rows are whole multiples of 256 only what HBM bounds gains: 256 x 200 x 200
+//    1.03, 512 x 200 x 200 1.07; 256 x 128 x 128 0.88, 512 x 128 x 128 0.91;
+//  - whole lines, Haar or 16 bits: 224 x 64 x 64 1.14 (BF16 linear), 160 x 128 x 128
+//    1.25 (Haar), 192 x 128 x 128 1.15 and 1.19; 192 x 64 x 64 0.92 (BF16 linear); a share
+//    of 5, 320 x 128 x 128 1.09 (BF16 linear) and 0.87 (Haar), of 4, 128 x 128 x 128 0.81
+//    and 0.91.
+static bool fwt3_wide(const FlFrameDesc& f, int nf, size_t esz)
+{
+    if (f.nx % 4) return false;
+    const int share = 2 * ((f.nx + 63) / 64) / ((f.nx + 255) / 256);
+    const size_t n = (size_t)f.nx * f.ny * f.nz, band = (size_t)nf * nf * nf * esz;
+    if (f.nx * esz % 64) return n * band >= ((size_t)16 << 20) && share >= (band <= 16 ? 6 : 4);
+    if (band > 64) return share >= 7 && (f.nx % 256 ? n >= 2000000 : n * band >= ((size_t)1 << 30));
+    return share >= 7 ? n >= 900000 : share == 6 ? n >= 1250000 : share == 5 && band > 32 && n >= 4000000;
+}
+
 template <typename XT, typename CT>
 static hipError_t fwt_t(const FlFrameDesc& f, const void* u, void* C, int level, hipStream_t st)
 {
@@ -945,7 +971,7 @@ static hipError_t fwt_t(const FlFrameDesc& f, const void* u, void* C, int level,
                 const dim3 grid((unsigned)((f.nx + 63) / 64), (unsigned)((f.ny + 3) / 4),
                                 (unsigned)std::min(65535, f.nz - z0));
                 if constexpr (NT == 3) {
-                    if (near && step == 1 && f.nx % 4 == 0 && ((uintptr_t)u | (uintptr_t)C) % 16 == 0) {
+                    if (near && step == 1 && fwt3_wide(f, NF, sizeof(CT)) && ((uintptr_t)u | (uintptr_t)C) % 16 == 0) {
                         hipLaunchKernelGGL((k_fwt3v<NF, XT, CT>), dim3((unsigned)((f.nx + 255) / 256), grid.y, grid.z),
                                            dim3(256), 0, st, (const XT*)u, (CT*)C, f.nx, f.ny, f.nz, z0, T);
                         continue;

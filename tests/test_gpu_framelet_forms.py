@@ -1,5 +1,6 @@
-"""The 3D analysis of four neighbours a thread returns the bits of the form of one
-(which buffers off 16-byte alignment take), in every storage type."""
+"""Which form of a framelet transform a size takes, on both sides of each line;
+and the 3D analysis of four neighbours a thread returns the bits of the form of
+one (which buffers off 16-byte alignment take), in every storage type."""
 import ctypes as C
 
 import pytest
@@ -33,3 +34,28 @@ def test_forms_agree(gpu, nx, ny, nz, frame, ut, ct):
     _analysis(S.kind, shape, u, c)(st)
     _analysis(S.kind, shape, off, want)(st)
     assert torch.equal(c, want)
+
+
+# (nx, ny, nz, frame, coefficient type, four a thread): rows of no whole 64-byte
+# lines by size and by a row's share of working lanes, whole lines likewise
+ANALYSIS = [
+    (68, 48, 48, "linear", F32, True), (68, 47, 48, "linear", F32, False), (64, 96, 96, "linear", F32, False),
+    (60, 96, 96, "linear", F32, False), (500, 19, 17, "linear", F32, True), (260, 25, 24, "linear", F32, True),
+    (132, 50, 48, "linear", BF16, True), (132, 46, 48, "linear", BF16, False), (196, 75, 73, "haar", BF16, True),
+    (196, 74, 75, "haar", F16, True), (260, 75, 73, "haar", BF16, False), (100, 75, 73, "haar", F32, True),
+    (102, 75, 73, "haar", F32, False),
+    (208, 99, 98, "linear", F32, True), (208, 97, 98, "linear", F32, False), (192, 256, 256, "linear", F32, False),
+    (256, 199, 200, "linear", F32, True), (256, 128, 128, "linear", F32, False), (16, 192, 192, "linear", F32, False),
+    (256, 60, 59, "haar", F32, True), (256, 59, 59, "haar", BF16, False), (192, 81, 81, "haar", F32, True),
+    (192, 80, 81, "linear", BF16, False), (320, 112, 112, "linear", BF16, True), (320, 112, 112, "haar", F32, False),
+    (128, 128, 128, "linear", BF16, False),
+]
+
+
+@pytest.mark.parametrize("nx, ny, nz, frame, dtype, wide", ANALYSIS)
+def test_analysis_form(gpu, nx, ny, nz, frame, dtype, wide):
+    from framelab_amd.framelets import FrameletSystem
+    S, shape = FrameletSystem(3, frame, 1), (nz, ny, nx)
+    u, c = torch.zeros(shape, device=gpu), torch.empty((S.nbands,) + shape, device=gpu, dtype=dtype)
+    names = captured_kernels(_analysis(S.kind, shape, u, c))
+    assert len(names) == 1 and ("k_fwt3v" in names[0]) == wide
