@@ -554,7 +554,9 @@ __global__ __launch_bounds__(4 * TXW) void k_iwt3m(const CT* __restrict__ C, XT*
 // halo: the taps wrap inside the tile), else 64-wide tiles.  Output slices
 // per workgroup: the longest run (fewer halo re-reads) that still gives at
 // least one workgroup per CU and `min_waves` waves, at least 4; fewer where not
-// even those give a workgroup per CU (64^3, linear: 66 -> 34 us).
+// even those give a workgroup per CU (64^3, linear: 66 -> 34 us), but of the 256-wide
+// tiles, one of which fills a CU, no more than the CUs (256 x 96 x 96, linear: 144
+// workgroups 98 us, 288 of half the run 132).
 template <int NF, int NT, int STEP, typename CT, typename XT>
 static void launch_iwt3m(const FlFrameDesc& f, const CT* C, XT* u, const FlTaps& T, float alpha, float beta,
                          const float* base, const CT* lp, hipStream_t st)
@@ -564,11 +566,12 @@ static void launch_iwt3m(const FlFrameDesc& f, const CT* C, XT* u, const FlTaps&
         constexpr int TY = ImGeom<NT, STEP, TXW>::TY;
         const unsigned tiles = (unsigned)(((f.nx + TXW - 1) / TXW) * ((f.ny + TY - 1) / TY));
         const size_t min_groups = std::max<size_t>(256, (size_t)FL_IWT_MIN_WAVES / (TXW / 16));
+        auto groups = [&](int run) { return (size_t)tiles * ((f.nz + run - 1) / run); };
         int zs = 64;
-        while (zs > 4 && (size_t)tiles * ((f.nz + zs - 1) / zs) < min_groups) zs /= 2;
-        while (zs > 1 && (size_t)tiles * ((f.nz + zs - 1) / zs) < 256) zs /= 2;
+        while (zs > 4 && groups(zs) < min_groups) zs /= 2;
+        while (zs > 1 && groups(zs) < 256 && (TXW == 64 || groups(zs / 2) <= 256)) zs /= 2;
         zs = std::min(zs, std::max(f.nz, 1));
-        const dim3 grid(tiles * (unsigned)((f.nz + zs - 1) / zs));
+        const dim3 grid((unsigned)groups(zs));
         hipLaunchKernelGGL((k_iwt3m<NF, NT, STEP, TXW, CT, XT>), grid, dim3(4 * TXW), 0, st, C, u, f.nx, f.ny, f.nz,
                            zs, T, alpha, beta, base, lp);
     };

@@ -30,7 +30,12 @@ def _hip():
 
 
 def captured_kernels(call):
-    """call(stream): launches on the stream it is given, allocating nothing."""
+    """Names; call(stream): launches on the stream it is given, allocating nothing."""
+    return [name for name, _ in captured_launches(call)]
+
+
+def captured_launches(call):
+    """As captured_kernels, with each launch's workgroups (x, y, z)."""
     hip = _hip()
 
     def ok(rc):
@@ -49,14 +54,14 @@ def captured_kernels(call):
         ok(hip.hipGraphGetNodes(graph, None, C.byref(n)))
         nodes = (C.c_void_p * n.value)()
         ok(hip.hipGraphGetNodes(graph, nodes, C.byref(n)))
-        names = []
+        launches = []
         for node in nodes:
             kind, p = C.c_int(), _KernelParams()
             ok(hip.hipGraphNodeGetType(C.c_void_p(node), C.byref(kind)))
             if kind.value != _KERNEL_NODE:
                 continue
             ok(hip.hipGraphKernelNodeGetParams(C.c_void_p(node), C.byref(p)))
-            names.append(hip.hipKernelNameRefByPtr(p.func, None).decode())
-        return names
+            launches.append((hip.hipKernelNameRefByPtr(p.func, None).decode(), (p.grid.x, p.grid.y, p.grid.z)))
+        return launches
     finally:
         ok(hip.hipGraphDestroy(graph))

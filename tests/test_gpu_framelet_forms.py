@@ -6,7 +6,7 @@ import ctypes as C
 import pytest
 import torch
 
-from graph_kernels import captured_kernels
+from graph_kernels import captured_kernels, captured_launches
 
 pytestmark = pytest.mark.gpu
 
@@ -59,3 +59,21 @@ def test_analysis_form(gpu, nx, ny, nz, frame, dtype, wide):
     u, c = torch.zeros(shape, device=gpu), torch.empty((S.nbands,) + shape, device=gpu, dtype=dtype)
     names = captured_kernels(_analysis(S.kind, shape, u, c))
     assert len(names) == 1 and ("k_fwt3v" in names[0]) == wide
+
+
+def _synthesis(kind, shape, c, u):
+    from framelab_amd import _lib
+    nx, ny, nz = (tuple(reversed(shape)) + (1,))[:3]
+    return lambda st: _lib.check(_lib.lib().fl_framelet_adjoint(len(shape), kind, 1, nx, ny, nz, C.c_void_p(c.data_ptr()),
+                                                                _lib.FL_F32, C.c_void_p(u.data_ptr()), _lib.FL_F32, None, st))
+
+
+# runs of slices: no more workgroups of 256-wide tiles than CUs if not by whole runs
+@pytest.mark.parametrize("nx, ny, nz, groups", [(256, 96, 96, 144), (256, 64, 64, 256), (768, 64, 48, 144), (64, 64, 64, 256),
+                                                (192, 64, 48, 288)])
+def test_synthesis_runs(gpu, nx, ny, nz, groups):
+    from framelab_amd.framelets import FrameletSystem
+    S, shape = FrameletSystem(3, "linear", 1), (nz, ny, nx)
+    c, u = torch.zeros((S.nbands,) + shape, device=gpu), torch.empty(shape, device=gpu)
+    (name, grid), = captured_launches(_synthesis(S.kind, shape, c, u))
+    assert "k_iwt3m" in name and grid == (groups, 1, 1)
