@@ -691,7 +691,11 @@ __global__ __launch_bounds__(TXW) void k_iwt2m(const CT* __restrict__ C, XT* u, 
 }
 
 // Launch of the 2D synthesis: one-wave tiles while the halo leaves them half
-// their columns, tiles of four waves while it leaves those, the gather beyond.
+// their columns, tiles of four waves while it leaves those, the gather beyond;
+// and for Haar images whose coefficients the caches hold, of which the gather
+// reads 36 a pixel (level 1, 2, 3, 5; gather against march, us: 1024 x 1024 9 and
+// 10, 18 and 22, 25 and 33, 43 and 57; 512 x 512 9, 13, 16, 21 and 9, 13, 16, 27; 1280 x
+// 1280 16 and 12, 32 and 24, 44 and 36, 69 and 63).
 // Rows per workgroup: 16, fewer where that leaves under 768 waves (1001 x 777
 // cubic, two levels: 16 rows 28 + 26 us, 8 rows 32 + 28, 4 rows 45 + 37; 512 x
 // 512: alike; 2048 x 2048: 32 rows 119 us, 64 rows 144).
@@ -710,8 +714,9 @@ static void launch_iwt2(const FlFrameDesc& f, const CT* C, XT* u, int step, cons
                            f.ny, step, rc, T, alpha, beta, base, lp);
     };
     const size_t rows = (size_t)f.ny + (size_t)step * 64;   // bounds the launch's second dimension
-    if (4 * h <= 64 && rows / 4 <= 65535) go(std::integral_constant<int, 64>{});
-    else if (4 * h <= 256 && rows / 4 <= 65535) go(std::integral_constant<int, 256>{});
+    const bool gather = NF == 2 && (size_t)f.nx * f.ny < 1300000;
+    if (!gather && 4 * h <= 64 && rows / 4 <= 65535) go(std::integral_constant<int, 64>{});
+    else if (!gather && 4 * h <= 256 && rows / 4 <= 65535) go(std::integral_constant<int, 256>{});
     else
         hipLaunchKernelGGL((k_iwt2<NF, NT, CT, XT>), dim3((unsigned)(((size_t)f.nx * f.ny + 255) / 256)), dim3(256), 0, st, C, u,
                            f.nx, f.ny, step, T, alpha, beta, base, lp);

@@ -77,3 +77,22 @@ def test_synthesis_runs(gpu, nx, ny, nz, groups):
     c, u = torch.zeros((S.nbands,) + shape, device=gpu), torch.empty(shape, device=gpu)
     (name, grid), = captured_launches(_synthesis(S.kind, shape, c, u))
     assert "k_iwt3m" in name and grid == (groups, 1, 1)
+
+
+@pytest.mark.parametrize("nx, ny, frame, march", [(1300, 999, "haar", False), (1300, 1001, "haar", True), (64, 64, "linear", True),
+                                                  (64, 64, "cubic", True), (64, 64, "haar", False)])
+def test_synthesis_2d_form(gpu, nx, ny, frame, march):
+    from framelab_amd.framelets import FrameletSystem
+    S, shape = FrameletSystem(2, frame, 1), (ny, nx)
+    c, u = torch.zeros((S.nbands,) + shape, device=gpu), torch.empty(shape, device=gpu)
+    assert ["k_iwt2m" in n for n in captured_kernels(_synthesis(S.kind, shape, c, u))] == [march]
+
+
+@pytest.mark.parametrize("level", [1, 3])
+def test_synthesis_2d_march_haar(gpu, level):
+    """Haar images of the marching form's sizes, against its inverse property."""
+    from framelab_amd.framelets import FrameletSystem
+    S = FrameletSystem(2, "haar", level)
+    u = torch.rand((1019, 1303), generator=torch.Generator(gpu).manual_seed(2), device=gpu)
+    back = S.adjointTransform(S.forwardTransform(u).frameletArray)
+    assert float((back - u).norm() / u.norm()) < 2e-6
