@@ -90,7 +90,7 @@ __global__ __launch_bounds__(64) void k_bfwd(const float* __restrict__ X, float*
     }
 }
 
-// Items of the problems without the windowed form (fl_fan_adj.h).
+// Items of the problems that the windowed form does not serve (fl_fan_windowed).
 template <bool MATCHED>
 __global__ __launch_bounds__(64) void k_badj(const float* __restrict__ Y, float* __restrict__ X,
                                             const BDesc* __restrict__ D, const int* __restrict__ start, int P,
@@ -111,7 +111,7 @@ __global__ __launch_bounds__(64) void k_badj(const float* __restrict__ Y, float*
     }
 }
 
-// Items of the problems with the windowed form: one 8 x 8 tile per workgroup
+// Items of the problems that the windowed form serves: one 8 x 8 tile per workgroup
 // at a time, its views shared by FAN_W waves.
 template <class Kind>
 __global__ __launch_bounds__(64 * (FAN_W + 1)) void k_badj_w(const float* __restrict__ Y, float* __restrict__ X,
@@ -367,9 +367,10 @@ struct fl_batch_s {
     std::vector<BDesc> desc;
     std::vector<long long> voff, soff;   // P+1 each
     BDesc* d_desc = nullptr;
-    // first items per problem; adjoint items split by form (general, windowed)
-    int *d_fstart = nullptr, *d_astart = nullptr, *d_wstart = nullptr, *d_vstart = nullptr;
-    int fwd_total = 0, adj_total = 0, adjw_total = 0, vec_total = 0;
+    // first items per problem; adjoint items split by form (general, windowed),
+    // of the exact and of the matched adjoint
+    int *d_fstart = nullptr, *d_astart[2] = {}, *d_wstart[2] = {}, *d_vstart = nullptr;
+    int fwd_total = 0, adj_total[2] = {}, adjw_total[2] = {}, vec_total = 0;
     int T = 64;                          // rays per forward item
     int fwd_grid = 0, adj_grid = 0, vec_grid = 0;
     // solver workspace
@@ -424,7 +425,8 @@ static int b_rebuild_fwd_table(fl_batch_s* B)
 static void b_free(fl_batch_s* B)
 {
     for (fl_plan pl : B->plans) fl_plan_destroy(pl);
-    void* ptrs[] = {B->d_desc, B->d_fstart, B->d_astart, B->d_wstart, B->d_vstart, B->r, B->p, B->q, B->sino, B->u, B->part,
+    void* ptrs[] = {B->d_desc, B->d_fstart, B->d_astart[0], B->d_astart[1], B->d_wstart[0], B->d_wstart[1],
+                    B->d_vstart, B->r, B->p, B->q, B->sino, B->u, B->part,
                     B->st, B->log, B->V, B->Dc, B->Atf, B->b};
     for (void* q : ptrs)
         if (q) (void)hipFree(q);
@@ -456,7 +458,7 @@ extern "C" int fl_batch_create(fl_batch* out, int nprob, const fl_geometry* geom
     (void)hipDeviceGetAttribute(&B->cus, hipDeviceAttributeMultiprocessorCount, B->device);
     B->voff.assign(nprob + 1, 0);
     B->soff.assign(nprob + 1, 0);
-    std::vector<int> as(nprob + 1, 0), ws(nprob + 1, 0), vs(nprob + 1, 0);
+    std::vector<int> vs(nprob + 1, 0);
     for (int i = 0; i < nprob; i++) {
         const fl_geometry& g = geoms[i];
         fl_plan pl = nullptr;
@@ -481,23 +483,31 @@ extern "C" int fl_batch_create(fl_batch* out, int nprob, const fl_geometry* geom
         d.n = (int)pl->nvox;
         B->voff[i + 1] = B->voff[i] + pl->nvox;
         B->soff[i + 1] = B->soff[i] + pl->ndet * pl->nv;
-        const int tiles = ((g.nx + 7) / 8) * ((g.ny + 7) / 8);
-        as[i + 1] = as[i] + (d.a.fan_cells ? 0 : tiles);
-        ws[i + 1] = ws[i] + (d.a.fan_cells ? tiles : 0);
         vs[i + 1] = vs[i] + (int)((pl->nvox + CH - 1) / CH);
         d.vec0 = vs[i];
         B->desc.push_back(d);
     }
-    B->adj_total = as[nprob];
-    B->adjw_total = ws[nprob];
     B->vec_total = vs[nprob];
     hipError_t e = hipMalloc((void**)&B->d_desc, nprob * sizeof(BDesc));
     if (e == hipSuccess) e = hipMalloc((void**)&B->d_fstart, (nprob + 1) * sizeof(int));
-    if (e == hipSuccess) e = hipMalloc((void**)&B->d_astart, (nprob + 1) * sizeof(int));
-    if (e == hipSuccess) e = hipMalloc((void**)&B->d_wstart, (nprob + 1) * sizeof(int));
     if (e == hipSuccess) e = hipMalloc((void**)&B->d_vstart, (nprob + 1) * sizeof(int));
-    if (e == hipSuccess) e = hipMemcpy(B->d_astart, as.data(), as.size() * sizeof(int), hipMemcpyHostToDevice);
-    if (e == hipSuccess) e = hipMemcpy(B->d_wstart, ws.data(), ws.size() * sizeof(int), hipMemcpyHostToDevice);
+    auto tiles = [&](int i) { return ((B->desc[i].f.nx + 7) / 8) * ((B->desc[i].f.ny + 7) / 8); };
+    long long all = 0;
+    for (int i = 0; i < nprob; i++) all += tiles(i);
+    for (int m = 0; m < 2 && e == hipSuccess; m++) {
+        std::vector<int> as(nprob + 1, 0), ws(nprob + 1, 0);
+        for (int i = 0; i < nprob; i++) {
+            const bool windowed = fl_fan_windowed(B->desc[i].a, m == 1, all);
+            as[i + 1] = as[i] + (windowed ? 0 : tiles(i));
+            ws[i + 1] = ws[i] + (windowed ? tiles(i) : 0);
+        }
+        B->adj_total[m] = as[nprob];
+        B->adjw_total[m] = ws[nprob];
+        e = hipMalloc((void**)&B->d_astart[m], as.size() * sizeof(int));
+        if (e == hipSuccess) e = hipMalloc((void**)&B->d_wstart[m], ws.size() * sizeof(int));
+        if (e == hipSuccess) e = hipMemcpy(B->d_astart[m], as.data(), as.size() * sizeof(int), hipMemcpyHostToDevice);
+        if (e == hipSuccess) e = hipMemcpy(B->d_wstart[m], ws.data(), ws.size() * sizeof(int), hipMemcpyHostToDevice);
+    }
     if (e == hipSuccess) e = hipMemcpy(B->d_vstart, vs.data(), vs.size() * sizeof(int), hipMemcpyHostToDevice);
     if (e == hipSuccess) e = hipStreamCreateWithFlags(&B->stream, hipStreamNonBlocking);
     if (e == hipSuccess) e = hipEventCreateWithFlags(&B->ev_in, hipEventDisableTiming);
@@ -553,19 +563,18 @@ static int b_forward(fl_batch_s* B, const float* x, float* y, bool gao, hipStrea
 
 static int b_adjoint(fl_batch_s* B, const float* y, float* x, bool matched, hipStream_t st)
 {
-    if (B->adjw_total) {
-        const dim3 gw((unsigned)std::min(B->adj_grid, B->adjw_total)), bw(64 * (FAN_W + 1));
-        if (matched)
-            hipLaunchKernelGGL(k_badj_w<FanMatched>, gw, bw, 0, st, y, x, B->d_desc, B->d_wstart, B->P, B->adjw_total);
-        else
-            hipLaunchKernelGGL(k_badj_w<FanExact>, gw, bw, 0, st, y, x, B->d_desc, B->d_wstart, B->P, B->adjw_total);
+    const int* astart = B->d_astart[matched];
+    const int* wstart = B->d_wstart[matched];
+    const int total = B->adj_total[matched], wtotal = B->adjw_total[matched];
+    if (wtotal) {
+        const dim3 gw((unsigned)std::min(B->adj_grid, wtotal)), bw(64 * (FAN_W + 1));
+        if (matched) hipLaunchKernelGGL(k_badj_w<FanMatched>, gw, bw, 0, st, y, x, B->d_desc, wstart, B->P, wtotal);
+        else hipLaunchKernelGGL(k_badj_w<FanExact>, gw, bw, 0, st, y, x, B->d_desc, wstart, B->P, wtotal);
     }
-    if (B->adj_total) {
-        const dim3 g((unsigned)std::min(B->adj_grid, B->adj_total));
-        if (matched)
-            hipLaunchKernelGGL(k_badj<true>, g, dim3(64), 0, st, y, x, B->d_desc, B->d_astart, B->P, B->adj_total);
-        else
-            hipLaunchKernelGGL(k_badj<false>, g, dim3(64), 0, st, y, x, B->d_desc, B->d_astart, B->P, B->adj_total);
+    if (total) {
+        const dim3 g((unsigned)std::min(B->adj_grid, total));
+        if (matched) hipLaunchKernelGGL(k_badj<true>, g, dim3(64), 0, st, y, x, B->d_desc, astart, B->P, total);
+        else hipLaunchKernelGGL(k_badj<false>, g, dim3(64), 0, st, y, x, B->d_desc, astart, B->P, total);
     }
     BCHK(hipGetLastError());
     return FL_OK;

@@ -185,6 +185,27 @@ __device__ __forceinline__ float fl_fan_adj_tile(const YT* __restrict__ Y, const
 constexpr int FAN_W = 7;
 constexpr int fl_fan_vb(int S) { return S <= 2 ? 4 : S <= 4 ? 2 : 1; }
 
+// Whether the windowed form serves a plan, `tiles` of 8 x 8 pixels in its launch.
+// It takes views by batches of FAN_W * fl_fan_vb(S), whole ones however few they
+// are, and pays for the first batch's start; the general form takes a lane's
+// views one by one, which is the shorter where tiles fill the chip by
+// themselves and views are few.  512 x 512 (4096 tiles) and 1024 x 1024, us, general
+// and windowed: exact, S = 2, 16 views 16 and 17, 41 and 58; 24 views 21 and 17, 58 and
+// 59; S = 4, 8 views 13 and 14, 36 and 46; 12 views 17 and 14, 51 and 47; matched, S = 2,
+// 8 views 18 and 23, 52 and 78; 16 views 34 and 22, 100 and 76; S = 4, 4 views 13 and 17,
+// 34 and 57; 8 views 21 and 17, 65 and 60.  384 x 384 (2304 tiles), 960 cells: exact, 3
+// views 7.4 and 9.0, 6 views 9.4 and 8.8; 256 x 256 (1024 tiles): within 7% from one view on.
+// In a batch, 8 x 512 x 512: exact, S = 2, 8 views 76 and 172, 20 views 181 and 181.
+inline bool fl_fan_windowed(const AdjGeom& g, bool matched, long long tiles)
+{
+    const int S = g.fan_cells;
+    if (S == 0 || tiles < 2048) return S != 0;
+    const int nv = g.tmp_size, per = FAN_W * fl_fan_vb(S), batches = (nv + per - 1) / per;
+    const int few = matched ? (S <= 2 ? 2 + 8 * batches : S <= 3 ? 3 + 4 * batches : S <= 4 ? 1 + 5 * batches : 1 + 2 * batches)
+                            : (S <= 2 ? 5 + 13 * batches : S <= 3 ? 6 + 6 * batches : S <= 4 ? 4 + 5 * batches : 3 + 2 * batches);
+    return nv > (tiles < 4096 ? few / 2 : few);
+}
+
 // 512 x 512 pixels, 640 views x 491 cells (S = 2), exact: 0.64 -> 0.26 ms;
 // 256 x 256, 360 x 512 (S = 4): 0.32 -> 0.059 ms (one lane per pixel and the
 // reference's window before).  Three producer waves 0.28 and 0.072 ms,
@@ -201,7 +222,7 @@ __global__ __launch_bounds__(64 * (FAN_W + 1)) void k_adj_fan_w(const YT* __rest
         fl_store(X, (size_t)it * g.nvox + (size_t)iy * g.nx + ix, v);
 }
 
-// Launches the windowed adjoint where the plan has one (true).
+// Launches the windowed adjoint where it serves the plan (true).
 template <class Kind, typename YT, typename XT>
 static bool fl_launch_fan_adj_w(const YT* Y, XT* X, const FwdGeom& f, const AdjGeom& g, hipStream_t st)
 {
@@ -210,6 +231,7 @@ static bool fl_launch_fan_adj_w(const YT* Y, XT* X, const FwdGeom& f, const AdjG
                            dim3((g.nx + 7) / 8, (g.ny + 7) / 8, g.nt), dim3(64 * (FAN_W + 1)), 0, st, Y, X, f, g);
         return true;
     };
+    if (!fl_fan_windowed(g, Kind::matched, (long long)((g.nx + 7) / 8) * ((g.ny + 7) / 8) * g.nt)) return false;
     switch (g.fan_cells) {
     case 2: return go(std::integral_constant<int, 2>{});
     case 3: return go(std::integral_constant<int, 3>{});

@@ -89,3 +89,35 @@ def test_batch_mixes_forms(gpu, oracle):
     for kind, k in ((ADJ_EXACT, 1), (ADJ_MATCHED, 2)):
         for got, r in zip(B.unpack(B.adjoint(y, kind=kind).cpu()), ref):
             assert bits_equal(got.numpy().ravel(), r[k])
+
+
+def _names(call):
+    from framelab_amd import _lib
+    from graph_kernels import captured_kernels
+    return captured_kernels(lambda st: _lib.check(call(_lib.lib(), st)))
+
+
+# (pixels a side, bins, views, exact windowed, matched windowed)
+@pytest.mark.parametrize("n, nd, nv, exact, matched", [(512, 512, 2, False, False), (512, 512, 15, False, True),
+                                                       (512, 512, 25, True, True), (512, 1024, 5, False, False),
+                                                       (512, 1024, 9, False, True), (512, 1024, 10, True, True),
+                                                       (512, 512, 30, False, True), (360, 360, 2, True, True),
+                                                       (384, 960, 3, False, False), (384, 960, 5, True, True)])
+def test_few_views(gpu, oracle, n, nd, nv, exact, matched):
+    """Images whose tiles fill the chip take the general form for few views, alone
+    and in a batch (one problem here: the same count of tiles)."""
+    from framelab_amd.batch import ProjectorBatch
+    from framelab_amd.projector import ADJ_EXACT, ADJ_MATCHED, Projector
+    p = _para((n, n, nd, nv))
+    P, B = Projector(p), ProjectorBatch([p])
+    y = torch.from_numpy(np.random.default_rng(n).standard_normal((nv, nd)).astype(np.float32)).to(gpu)
+    x = torch.empty(P.vol_shape, device=gpu)
+    for kind, windowed in ((ADJ_EXACT, exact), (ADJ_MATCHED, matched)):
+        one = _names(lambda L, st: L.fl_adjoint(P.handle, y.data_ptr(), 0, x.data_ptr(), 0, kind, st))
+        many = _names(lambda L, st: L.fl_batch_adjoint(B.handle, y.data_ptr(), x.data_ptr(), kind, st))
+        assert ["k_adj_fan_w" in k for k in one] == ["k_badj_w" in k for k in many] == [windowed]
+        got = P.adjoint(y, kind=kind)
+        assert torch.equal(B.adjoint(y.ravel(), kind=kind), got.ravel())
+    want = oracle.atx_fan_f32(y.cpu().numpy().ravel(), p)
+    got = P.adjoint(y).cpu().numpy().ravel()
+    assert bits_equal(got, want), first_mismatch(got, want)
