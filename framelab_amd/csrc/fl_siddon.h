@@ -90,18 +90,54 @@ FL_HD float sid_div(float num, float d, float r)
     return fmaf(e, r, q);
 }
 
+// floor to int in one instruction (saturating, 0 for NaN, as floorf and the
+// conversion, which the compiler keeps apart).
+FL_HD int sid_floor(float v)
+{
+#if defined(__HIP_DEVICE_COMPILE__)
+    int r;
+    asm("v_cvt_flr_i32_f32 %0, %1" : "=v"(r) : "v"(v));
+    return r;
+#else
+    return (int)floorf(v);
+#endif
+}
+
+// fminf in one instruction: of operands whose origin the compiler cannot see it
+// quiets each one first.
+FL_HD float sid_min(float a, float b)
+{
+#if defined(__HIP_DEVICE_COMPILE__)
+    float r;
+    asm("v_min_f32 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+    return r;
+#else
+    return fminf(a, b);
+#endif
+}
+FL_HD float sid_min3(float a, float b, float c)
+{
+#if defined(__HIP_DEVICE_COMPILE__)
+    float r;
+    asm("v_min3_f32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
+    return r;
+#else
+    return fminf(fminf(a, b), c);
+#endif
+}
+
 // Cell index of the midpoint along an x/y axis: floor(o + m*d + n/2).
 FL_HD int sid_cell_xy(const SidAxis& a, float m)
 {
     float t = a.o + m * a.d;
-    return (int)floorf(t + (float)a.nh);
+    return sid_floor(t + (float)a.nh);
 }
 // z axis: floor((o + m*d)/dz0 + n/2); dz0 == 1 divides exactly, so it is skipped.
 FL_HD int sid_cell_z(const SidAxis& a, float m, bool dz_one)
 {
     float t = a.o + m * a.d;
     if (!dz_one) t = t / a.s;
-    return (int)floorf(t + (float)a.nh);
+    return sid_floor(t + (float)a.nh);
 }
 
 FL_HD bool sid_in(const SidAxis& a, int t) { return (unsigned)t < (unsigned)a.n; }
@@ -202,18 +238,6 @@ FL_HD bool sid_start(const SidAxis& ax, const SidAxis& ay, const SidAxis& az, Si
     return true;
 }
 
-// floor to int in one instruction (the walks' midpoints are never NaN).
-FL_HD int sid_floor(float v)
-{
-#if defined(__HIP_DEVICE_COMPILE__)
-    int r;
-    asm("v_cvt_flr_i32_f32 %0, %1" : "=v"(r) : "v"(v));
-    return r;
-#else
-    return (int)floorf(v);
-#endif
-}
-
 // Generic walk over one ray.  The visitor receives (linear voxel index
 // (z*ny+y)*nx+x, alpha difference of the segment) for every in-volume segment
 // in traversal order; the length is that difference times |d|.
@@ -228,8 +252,7 @@ FL_HD void sid_walk_t(const SidAxis& ax, const SidAxis& ay, const SidAxis& az, f
 
     const int nx = ax.n, ny = ay.n;
     for (;;) {
-        float an = fminf(qx.a, qy.a);
-        if (NZ3) an = fminf(an, qz.a);
+        const float an = NZ3 ? sid_min3(qx.a, qy.a, qz.a) : sid_min(qx.a, qy.a);
         if (an == FL_INF) break;
         float m = (cur + an) * 0.5f;
         int tx = sid_cell_xy(ax, m);
@@ -238,7 +261,7 @@ FL_HD void sid_walk_t(const SidAxis& ax, const SidAxis& ay, const SidAxis& az, f
         if (NZ3) {
             float t = az.o + m * az.d;
             if (!DZ1) t = sid_div(t, az.s, rs);
-            tz = (int)floorf(t + (float)az.nh);
+            tz = sid_floor(t + (float)az.nh);
         }
         bool in = sid_in(ax, tx) && sid_in(ay, ty) && (!NZ3 || sid_in(az, tz));
         if constexpr (ALL) {

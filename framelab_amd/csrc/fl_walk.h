@@ -240,7 +240,7 @@ __device__ __forceinline__ float walk_rays(WalkAxis& X, WalkAxis& Y, WalkAxis& Z
     };
     auto far = [&](int tx, int ty, int tz) { return sid_far(ax, tx) || sid_far(ay, ty) || (NZ3 && sid_far(az, tz)); };
     auto near = [&](int tx, int ty, int tz) { return sid_near(ax, tx) || sid_near(ay, ty) || (NZ3 && sid_near(az, tz)); };
-    auto next = [&] { return NZ3 ? fminf(fminf(X.a, Y.a), Z.a) : fminf(X.a, Y.a); };
+    auto next = [&] { return NZ3 ? sid_min3(X.a, Y.a, Z.a) : sid_min(X.a, Y.a); };
     auto read = [&](unsigned off) { return fl_raw((const VT*)((const char*)vol + off)); };
     auto value = [&](decltype(read(0u)) r) { return fl_unraw((const VT*)nullptr, r); };
     float acc = 0.0f;
@@ -330,7 +330,8 @@ __device__ __forceinline__ float walk_rays(WalkAxis& X, WalkAxis& Y, WalkAxis& Z
     // run: still walking (without a plane ahead there is nothing to walk).  A
     // lane that has finished gets NaN plane parameters: it crosses nothing, and
     // whatever is computed from them is masked by run or ran.  (Lane masks, so
-    // that the tests of a batch are scalar.)
+    // that the tests of a batch are scalar.)  Compiled with NaN semantics; the
+    // mins are written out (sid_min), which cost as little as without.
     uint64_t run = __builtin_amdgcn_ballot_w64(live && next() < FL_INF);
     float nan;
     asm volatile("v_mov_b32_e32 %0, 0x7fc00000" : "=v"(nan));
@@ -348,14 +349,16 @@ __device__ __forceinline__ float walk_rays(WalkAxis& X, WalkAxis& Y, WalkAxis& Z
     const uint64_t all = __builtin_amdgcn_read_exec();
     auto issue = [&](Batch& t) {
         const float from = cur;
-        float an[D], dmin = FL_INF;
+        float an[D], dmin = FL_INF, even = 0.0f;
 #pragma unroll
         for (int u = 0; u < D; u++) {
             an[u] = next();
             const float dal = an[u] - cur;
             t.S[u] = dal * L;
             t.x[u] = read(lay.place(X.f, Y.f, Z.f));
-            dmin = fminf(dmin, dal);
+            if (u % 2 == 1) dmin = sid_min3(dmin, even, dal);
+            else if (u == D - 1) dmin = sid_min(dmin, dal);
+            else even = dal;
             walk_cross<true, UNIFORM, Layout::MASKED>(X, an[u], lay.mx, all);
             walk_cross<true, UNIFORM, Layout::MASKED>(Y, an[u], lay.my, all);
             if constexpr (NZ3) walk_cross<DZ1, UNIFORM, Layout::MASKED>(Z, an[u], lay.mz, all);
