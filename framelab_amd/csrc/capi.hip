@@ -81,9 +81,10 @@ static void plan_free_arrays(fl_plan_s* p)
     if (p->fwd_done) (void)hipEventDestroy(p->fwd_done);
 }
 
-// Forwards of one plan share its brick buffer, so each is ordered
+// Forwards of one plan share its brick buffer, so each that uses it is ordered
 // after the previous one, whatever streams they run on: wait for the event
-// the previous forward recorded, record it again after this one.  A stream
+// the previous forward recorded, record it again after this one (a fan
+// forward that would wait takes no bricks: fl_bricks_busy).  A stream
 // under graph capture is left alone (external events cannot enter a
 // capture); the solvers that capture forwards order their private stream
 // against the caller's, and a fan forward that anyone else captures takes no
@@ -106,7 +107,28 @@ static int fwd_order_end(fl_plan_s* p, hipStream_t st, bool order)
     const hipError_t e = hipEventRecord(p->fwd_done, st);
     if (e != hipSuccess) return fl_hip_fail(e, "forward ordering");
     p->fwd_pending = true;
+    p->fwd_stream = p->fwd_after = st;
     return FL_OK;
+}
+
+// Fan forwards on several streams need not wait for one another: the image as
+// it is gives the same bits as its bricks.  (The query is made in relaxed
+// capture mode, so that it is allowed while some other stream is captured.)
+bool fl_bricks_busy(fl_plan_s* p, hipStream_t st)
+{
+    if (p->cone || !p->fwd_pending || st == p->fwd_stream || st == p->fwd_after) return false;
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+    const bool relaxed = hipThreadExchangeStreamCaptureMode(&mode) == hipSuccess;
+    const bool busy = hipEventQuery(p->fwd_done) != hipSuccess;
+    if (busy) (void)hipGetLastError();   // hipErrorNotReady
+    if (relaxed) (void)hipThreadExchangeStreamCaptureMode(&mode);
+    return busy;
+}
+
+void fl_bricks_ordered(fl_plan_s* p, hipStream_t earlier, hipStream_t later)
+{
+    std::lock_guard<std::mutex> lk(p->fwd_mu);
+    if (later != p->fwd_stream && (earlier == p->fwd_stream || earlier == p->fwd_after)) p->fwd_after = later;
 }
 
 // AdjGeom::win_ref for a cone plan: whether the reference's detector window
@@ -611,17 +633,19 @@ int fl_forward_ordered(fl_plan_s* p, const void* d_x, int xt, void* d_y, int yt,
         if (e == hipErrorInvalidValue) return fl_fail(FL_ERR_UNSUPPORTED, "dtype combination %d/%d", xt, yt);
         return e == hipSuccess ? FL_OK : fl_hip_fail(e, "forward launch");
     };
-    // a fan forward captured by someone else replays in no order with the
-    // plan's other forwards: it reads its image as it is
-    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
-    if (!p->cone && p->d_bricks && !owns_capture && hipStreamIsCapturing(st, &cs) != hipSuccess) cs = hipStreamCaptureStatusActive;
-    if (!p->d_bricks || cs != hipStreamCaptureStatusNone) {
+    auto as_it_is = [&] {
         FwdGeom g = p->fg;
         g.tracked = false;
         const int rc = launch(g);
         return rc ? rc : fl_ok();
-    }
+    };
+    // a fan forward captured by someone else replays in no order with the
+    // plan's other forwards: it reads its image as it is
+    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+    if (!p->cone && p->d_bricks && !owns_capture && hipStreamIsCapturing(st, &cs) != hipSuccess) cs = hipStreamCaptureStatusActive;
+    if (!p->d_bricks || cs != hipStreamCaptureStatusNone) return as_it_is();
     std::lock_guard<std::mutex> lk(p->fwd_mu);
+    if (!owns_capture && fl_bricks_busy(p, st)) return as_it_is();
     bool order = false;
     int rc = fwd_order_begin(p, st, order);
     if (!rc) rc = launch(p->fg);

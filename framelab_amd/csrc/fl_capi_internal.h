@@ -27,6 +27,8 @@ struct fl_plan_s {
     // whatever stream it ran) through this event, recorded after it
     hipEvent_t fwd_done = nullptr;
     bool fwd_pending = false;
+    // the stream it was recorded on, and one that was ordered after it since
+    void *fwd_stream = nullptr, *fwd_after = nullptr;
     std::mutex fwd_mu;
     // fan, finite-width beam: strip lines per (view, cell, edge) and cell
     // edge tables (built on first use / uploaded when given)
@@ -58,6 +60,10 @@ size_t fl_tracked_frame_elems(int nx, int ny, int nz);
 size_t fl_fan_brick_elems(int nx, int ny);
 // fl_forward for a caller that orders its own captures against the plan's
 // other forwards (the solvers): captured fan forwards may use the plan's bricks
+// a fan plan's bricks are in use on a stream that st is not ordered after (fwd_mu held)
+bool fl_bricks_busy(fl_plan_s* p, hipStream_t st);
+// `later` was made to wait for `earlier`
+void fl_bricks_ordered(fl_plan_s* p, hipStream_t earlier, hipStream_t later);
 int fl_forward_ordered(fl_plan_s* p, const void* d_x, int xt, void* d_y, int yt, void* stream, bool owns_capture);
 // detector coordinates may stray from a uniform grid by at most this many
 // cells for the voxel-driven adjoints (their windows widen by 0.05 cells)

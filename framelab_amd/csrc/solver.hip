@@ -498,7 +498,8 @@ int cg_run(fl_plan_s* pl, Workspace& w, const float* b, float* u_caller, float l
     int rc;
     if ((rc = cg_init(pl, w, b, u, lam, flags, tol, st))) return rc;
     if (iters <= 0) return FL_OK;
-    if (flags & FL_SOLVE_GRAPH) {
+    bool replay = flags & FL_SOLVE_GRAPH;
+    if (replay) {
         const bool hit = w.gexec && w.gkey_lam == lam && w.gkey_flags == flags;
         if (!hit) {
             drop_graph(w);
@@ -519,33 +520,40 @@ int cg_run(fl_plan_s* pl, Workspace& w, const float* b, float* u_caller, float l
         // The captured forwards write the plan's brick buffer, and a stream
         // under capture takes no part in the plan's forward ordering: order
         // the replays after any forward in flight on another stream, and
-        // later forwards after the replays.
+        // later forwards after the replays.  (Of a fan plan the iterations run
+        // uncaptured instead, which need not wait for it.)
         std::lock_guard<std::mutex> lk(pl->fwd_mu);
-        if (pl->fwd_done && pl->fwd_pending) HIPCHK(hipStreamWaitEvent(st, pl->fwd_done, 0));
-        for (int k = 0; k < iters; k++) HIPCHK(hipGraphLaunch(w.gexec, st));
-        if (pl->fwd_done) {
-            HIPCHK(hipEventRecord(pl->fwd_done, st));
-            pl->fwd_pending = true;
+        replay = !fl_bricks_busy(pl, st);
+        if (replay) {
+            if (pl->fwd_done && pl->fwd_pending) HIPCHK(hipStreamWaitEvent(st, pl->fwd_done, 0));
+            for (int k = 0; k < iters; k++) HIPCHK(hipGraphLaunch(w.gexec, st));
+            if (pl->fwd_done) {
+                HIPCHK(hipEventRecord(pl->fwd_done, st));
+                pl->fwd_pending = true;
+                pl->fwd_stream = pl->fwd_after = st;
+            }
         }
-    } else {
+    }
+    if (!replay)
         for (int k = 0; k < iters; k++)
             if ((rc = cg_body(pl, w, u, lam, flags, st, false))) return rc;
-    }
     HIPCHK(fl_launch_copy(u, u_caller, n, st));
     return FL_OK;
 }
 
-int begin_on(Workspace& w, hipStream_t caller)
+int begin_on(fl_plan_s* pl, Workspace& w, hipStream_t caller)
 {
     HIPCHK(hipEventRecord(w.ev_in, caller));
     HIPCHK(hipStreamWaitEvent(w.stream, w.ev_in, 0));
+    fl_bricks_ordered(pl, caller, w.stream);
     return FL_OK;
 }
 
-int end_on(Workspace& w, hipStream_t caller)
+int end_on(fl_plan_s* pl, Workspace& w, hipStream_t caller)
 {
     HIPCHK(hipEventRecord(w.ev_out, w.stream));
     HIPCHK(hipStreamWaitEvent(caller, w.ev_out, 0));
+    fl_bricks_ordered(pl, w.stream, caller);
     return FL_OK;
 }
 
@@ -708,7 +716,7 @@ extern "C" int fl_cgls(fl_plan pl, const float* d_b, float* d_u, float lam, int 
     int rc;
     if ((rc = ensure_cg(pl, w, iters + 1, flags))) return rc;
     hipStream_t caller = (hipStream_t)stream;
-    if ((rc = begin_on(w, caller))) return rc;
+    if ((rc = begin_on(pl, w, caller))) return rc;
     if ((rc = cg_run(pl, w, d_b, d_u, lam, iters, tol, flags))) return rc;
     if (gamma_log || iters_done) {
         CgState s;
@@ -720,7 +728,7 @@ extern "C" int fl_cgls(fl_plan pl, const float* d_b, float* d_u, float lam, int 
         if (gamma_log)
             for (int k = s.iter + 1; k <= iters; k++) gamma_log[k] = s.gnext;
     }
-    if ((rc = end_on(w, caller))) return rc;
+    if ((rc = end_on(pl, w, caller))) return rc;
     return fl_ok();
 }
 
@@ -790,7 +798,7 @@ extern "C" int fl_split_bregman(fl_plan pl, int kind, int level, const float* d_
         w.res_n = (size_t)(outer > 0 ? outer : 1);
     }
     hipStream_t caller = (hipStream_t)stream, st = w.stream;
-    if ((rc = begin_on(w, caller))) return rc;
+    if ((rc = begin_on(pl, w, caller))) return rc;
     const int kind_adj = (flags & FL_SOLVE_MATCHED) ? FL_ADJ_MATCHED : FL_ADJ_EXACT;
     // v = alpha = W u0 (so alpha - v = 0 and b = Atf), Atf = A^T f
     for (int L = 1; L <= level; L++) {
@@ -836,7 +844,7 @@ extern "C" int fl_split_bregman(fl_plan pl, int kind, int level, const float* d_
         if (e != hipSuccess) rc = fl_hip_fail(e, "residual log");
     }
     if (rc) return rc;
-    if ((rc = end_on(w, caller))) return rc;
+    if ((rc = end_on(pl, w, caller))) return rc;
     return fl_ok();
 }
 
@@ -853,7 +861,7 @@ extern "C" int fl_grad_data(fl_plan pl, const float* d_x, const float* d_b, floa
     // the solvers: the gradient runs on the workspace stream, ordered after
     // the caller's stream and before the caller's later work
     hipStream_t caller = (hipStream_t)stream, st = w.stream;
-    if ((rc = begin_on(w, caller))) return rc;
+    if ((rc = begin_on(pl, w, caller))) return rc;
     const size_t ns = (size_t)pl->ndet * pl->nv;
     if ((rc = fl_forward(pl, d_x, FL_F32, w.sino, FL_F32, st))) return rc;
     const unsigned g = grid_for(ns);
@@ -867,7 +875,7 @@ extern "C" int fl_grad_data(fl_plan pl, const float* d_x, const float* d_b, floa
         HIPCHK(hipMemcpyAsync(loss, out, sizeof(double), hipMemcpyDeviceToHost, st));
         HIPCHK(hipStreamSynchronize(st));
     }
-    if ((rc = end_on(w, caller))) return rc;
+    if ((rc = end_on(pl, w, caller))) return rc;
     return fl_ok();
 }
 
