@@ -462,7 +462,7 @@ extern "C" int fl_batch_create(fl_batch* out, int nprob, const fl_geometry* geom
     for (int i = 0; i < nprob; i++) {
         const fl_geometry& g = geoms[i];
         fl_plan pl = nullptr;
-        int rc = fl_plan_create(&pl, &g);
+        int rc = fl_plan_create_with(&pl, &g, false);
         if (rc) {
             b_free(B);
             delete B;

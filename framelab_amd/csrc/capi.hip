@@ -230,7 +230,9 @@ static int fan_shadow_cells(const fl_geometry* g, double pa, double det_dev, con
     return n <= g->na && out.fan_tile <= 64 ? n : 0;
 }
 
-extern "C" int fl_plan_create(fl_plan* out, const fl_geometry* g)
+extern "C" int fl_plan_create(fl_plan* out, const fl_geometry* g) { return fl_plan_create_with(out, g, true); }
+
+int fl_plan_create_with(fl_plan* out, const fl_geometry* g, bool fan_bricks)
 {
     if (!out || !g) return fl_fail(FL_ERR_INVALID, "null plan or geometry");
     *out = nullptr;
@@ -408,7 +410,7 @@ extern "C" int fl_plan_create(fl_plan* out, const fl_geometry* g)
     // (8 us): 256 x 256, 256 views x 256 cells 40 us as it is, 48 from bricks;
     // 360 x 512 102 and 85; 384 x 384, 400 x 500 145 and 136; 1024 x 1024, 900 x
     // 1000 1176 and 925, 900 x 2000 1866 and 1313
-    const size_t fb = !cone && (size_t)g->nv * g->na >= 150000 ? fl_fan_brick_elems(g->nx, g->ny) : 0;
+    const size_t fb = !cone && fan_bricks && (size_t)g->nv * g->na >= 150000 ? fl_fan_brick_elems(g->nx, g->ny) : 0;
     if (!rc && fb) {
         p->fg.tracked = hipMalloc(&p->d_bricks, fb * (size_t)g->nt * 4) == hipSuccess;
         if (!p->fg.tracked) {
@@ -836,7 +838,7 @@ void frames_to_views(int nt, int nv, const int* id_Y, const int* Nv, int tmp, st
 int run_forward_host(const fl_geometry& g, const float* X, float* y, float* yNorm, bool gao, bool fb = false)
 {
     PlanGuard pg;
-    int rc = fl_plan_create(&pg.p, &g);
+    int rc = fl_plan_create_with(&pg.p, &g, !gao && !fb);
     if (rc) return rc;
     size_t nvox = (size_t)pg.p->nvox * g.nt, ny = (size_t)pg.p->ndet * g.nv;
     DevBuf dx, dy, dn;
@@ -861,7 +863,7 @@ int run_forward_host(const fl_geometry& g, const float* X, float* y, float* yNor
 int run_adjoint_host(const fl_geometry& g, const float* Y, float* X, int kind = FL_ADJ_EXACT)
 {
     PlanGuard pg;
-    int rc = fl_plan_create(&pg.p, &g);
+    int rc = fl_plan_create_with(&pg.p, &g, false);
     if (rc) return rc;
     size_t nvox = (size_t)pg.p->nvox * g.nt, ny = (size_t)pg.p->ndet * g.nv;
     DevBuf dx, dy;
