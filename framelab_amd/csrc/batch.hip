@@ -822,27 +822,43 @@ extern "C" int fl_batch_autotune(fl_batch B, int* fwd_tile, int* fwd_grid, int* 
     };
     if (!rc) {
         (void)hipMemsetAsync(x, 0, nv * 4, st);
+        // The grids in force first, then the candidates that launch a number of
+        // workgroups not yet timed: what is kept is never slower than what was.
+        const int T0 = B->T;
         float best = 1e30f;
-        int bT = B->T, bG = B->fwd_grid;
-        for (int T : {64, 128, 256}) {
+        int bT = T0, bG = B->fwd_grid;
+        auto grids = [&](int now, int total, std::initializer_list<int> per_cu, auto&& timed) {
+            std::vector<int> seen;
+            auto consider = [&](int grid) {
+                const int launched = std::min(grid, std::max(total, 1));
+                if (std::find(seen.begin(), seen.end(), launched) != seen.end()) return;
+                seen.push_back(launched);
+                timed(grid);
+            };
+            consider(now);
+            for (int m : per_cu) consider(m * B->cus);
+        };
+        const int G0 = B->fwd_grid;
+        for (int T : {T0, 64, 128, 256}) {
+            if (T == T0 && best < 1e30f) continue;
             B->T = T;
             if ((rc = b_rebuild_fwd_table(B))) break;
-            for (int m : {2, 4, 8, 16}) {
-                B->fwd_grid = m * B->cus;
-                float ms = time_it([&] { (void)b_forward(B, x, y, false, st); });
-                if (ms < best) { best = ms; bT = T; bG = B->fwd_grid; }
-            }
+            grids(G0, B->fwd_total, {2, 4, 8, 16, 32, 64}, [&](int grid) {
+                B->fwd_grid = grid;
+                const float ms = time_it([&] { (void)b_forward(B, x, y, false, st); });
+                if (ms < best) { best = ms; bT = T; bG = grid; }
+            });
         }
         B->T = bT;
         B->fwd_grid = bG;
         if (!rc) rc = b_rebuild_fwd_table(B);
         best = 1e30f;
         int bA = B->adj_grid;
-        for (int m : {2, 4, 8, 16}) {
-            B->adj_grid = m * B->cus;
-            float ms = time_it([&] { (void)b_adjoint(B, y, x, false, st); });
-            if (ms < best) { best = ms; bA = B->adj_grid; }
-        }
+        grids(bA, std::max(B->adj_total[0], B->adjw_total[0]), {2, 4, 8, 16, 32}, [&](int grid) {
+            B->adj_grid = grid;
+            const float ms = time_it([&] { (void)b_adjoint(B, y, x, false, st); });
+            if (ms < best) { best = ms; bA = grid; }
+        });
         B->adj_grid = bA;
         b_drop_graph(B);   // a captured iteration holds the old launch shapes
     }

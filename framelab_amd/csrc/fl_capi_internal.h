@@ -61,7 +61,6 @@ size_t fl_tracked_frame_elems(int nx, int ny, int nz);
 size_t fl_fan_brick_elems(int nx, int ny);
 // fl_plan_create, or a fan plan without bricks: the batches', whose forward reads
 // the packed images as they are, and those of drop-ins that make no Siddon forward
-// (256 x 256, 360 x 512, column walk: 0.56 -> 0.48 ms a call)
 int fl_plan_create_with(fl_plan* out, const fl_geometry* g, bool fan_bricks);
 // fl_forward for a caller that orders its own captures against the plan's
 // other forwards (the solvers): captured fan forwards may use the plan's bricks
