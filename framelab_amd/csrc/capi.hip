@@ -391,16 +391,14 @@ int fl_plan_create_with(fl_plan* out, const fl_geometry* g, bool fan_bricks)
     if (cone) {
         // the forward gathers from a bricked copy of its input (padded to
         // whole bricks of the largest layout; 4-byte elements cover every
-        // storage type).  The tracked walk's copy is padded to powers of two,
-        // up to four times the voxels: above 4 GiB it is taken only where it
-        // is at most twice the unpadded one, and only if there is room.
-        const size_t fr = fl_bricked_frame_elems(g->nx, g->ny, g->nz), tr = fl_tracked_frame_elems(g->nx, g->ny, g->nz);
-        const size_t want = std::max(fr, tr) * (size_t)g->nt * 4;
-        if (tr && (tr <= 2 * fr || want <= ((size_t)4 << 30))) {
-            p->fg.tracked = hipMalloc(&p->d_bricks, want) == hipSuccess;
+        // storage type), in the tracked walk's layout if there is room
+        const size_t tr = fl_cone_copy_bytes(g->nx, g->ny, g->nz, g->nt, true);
+        if (tr) {
+            p->fg.tracked = hipMalloc(&p->d_bricks, tr) == hipSuccess;
             if (!p->fg.tracked) (void)hipGetLastError();
         }
-        if (!p->fg.tracked && hipMalloc(&p->d_bricks, fr * (size_t)g->nt * 4) != hipSuccess) rc = fl_fail(FL_ERR_ALLOC, "brick buffer");
+        if (!p->fg.tracked && hipMalloc(&p->d_bricks, fl_cone_copy_bytes(g->nx, g->ny, g->nz, g->nt, false)) != hipSuccess)
+            rc = fl_fail(FL_ERR_ALLOC, "brick buffer");
         else if (hipEventCreateWithFlags(&p->fwd_done, hipEventDisableTiming) != hipSuccess)
             rc = fl_fail(FL_ERR_HIP, "forward ordering event");
     }

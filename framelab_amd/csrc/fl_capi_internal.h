@@ -55,9 +55,9 @@ struct fl_plan_s {
 };
 
 constexpr int FL_FWD_NTILES = 8;   // cone forward ray-tile shapes (siddon.hip)
-// elements of the largest bricked frame of any of them (siddon.hip)
-size_t fl_bricked_frame_elems(int nx, int ny, int nz);
-size_t fl_tracked_frame_elems(int nx, int ny, int nz);
+// bytes of a bricked copy of nt frames that serves all of them (siddon.hip); with
+// the tracked walk's layout, 0 where that is not to be used
+size_t fl_cone_copy_bytes(int nx, int ny, int nz, int nt, bool tracked);
 size_t fl_fan_brick_elems(int nx, int ny);
 // fl_plan_create, or a fan plan without bricks: the batches', whose forward reads
 // the packed images as they are, and those of drop-ins that make no Siddon forward

@@ -100,18 +100,29 @@ struct Bricks {
 };
 
 // Elements of the largest unpadded bricked frame of any launch shape.
-size_t fl_bricked_frame_elems(int nx, int ny, int nz)
+static size_t fl_bricked_frame_elems(int nx, int ny, int nz)
 {
     return std::max({Bricks<8, 8>(nx, ny, nz).frame, Bricks<4, 4, 4>(nx, ny, nz).frame, Bricks<4, 4, 2>(nx, ny, nz).frame});
 }
 
 // Elements of the tracked walk's padded frame; 0 where its 32-bit byte offsets
 // do not reach (2^30 voxels and more): such volumes take the unpadded bricks.
-size_t fl_tracked_frame_elems(int nx, int ny, int nz)
+static size_t fl_tracked_frame_elems(int nx, int ny, int nz)
 {
     if (nx >= (1 << 24) || ny >= (1 << 24) || nz >= (1 << 24)) return 0;
     const size_t frame = ConeBricks<4>(nx, ny).frame(nz);
     return frame <= ((size_t)1 << 30) ? frame : 0;
+}
+
+// The tracked walk's copy is padded to powers of two, up to four times the voxels
+// and more in thin volumes: above 4 GiB it is used only where it is at most twice
+// the unpadded one.
+size_t fl_cone_copy_bytes(int nx, int ny, int nz, int nt, bool tracked)
+{
+    const size_t fr = fl_bricked_frame_elems(nx, ny, nz), tr = fl_tracked_frame_elems(nx, ny, nz);
+    if (!tracked) return fr * (size_t)nt * 4;
+    const size_t want = std::max(fr, tr) * (size_t)nt * 4;
+    return tr && (tr <= 2 * fr || want <= ((size_t)4 << 30)) ? want : 0;
 }
 
 // Elements of a fan image's bricked copy, 0 where its 32-bit byte offsets do not
