@@ -162,12 +162,21 @@ FL_HD float fl_chord_box3_r(const float* p, const float* h, bool xmajor, const F
 }
 
 // sqrtf(s) for 2^-96 <= s < 2^96: one residual step on the hardware's reciprocal
-// square root.  Correctly rounded (every float of that range checked against
-// sqrtf) in five instructions.
+// square root.  Correctly rounded in five instructions: no theorem says so, but
+// every float of that range is checked against sqrtf on the device
+// (tests/diag/diag.hip).
 __device__ __forceinline__ float fl_sqrt_mid(float s)
 {
     const float y = __builtin_amdgcn_rsqf(s), r = s * y;
     return fmaf(fmaf(-r, r, s), 0.5f * y, r);
+}
+
+// 1/d, correctly rounded, for 2^-22 <= d <= 2: one Newton step on the hardware's
+// reciprocal (every float of that range is checked likewise).
+__device__ __forceinline__ float fl_rcp_mid(float d)
+{
+    const float r = __builtin_amdgcn_rcpf(d);
+    return fmaf(fmaf(-d, r, 1.0f), r, r);
 }
 
 // sqrtf(s) for finite s >= 0: the hardware square root and the

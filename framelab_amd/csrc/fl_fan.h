@@ -74,9 +74,8 @@ __device__ __forceinline__ float fl_fan_ray_sum(const VT* __restrict__ x, const 
 // skips is +0, which leaves a sum that starts at +0 unchanged.  A wave takes
 // GAO_WA cells of 16 / GAO_WA views.
 //
-// Divisions by the column's span d are Markstein quotients of one reciprocal:
-// one Newton step on the hardware's is 1/d correctly rounded for every mantissa
-// (all 2^23 checked at the exponents of a span, 2^-22 .. 2); the root's
+// Divisions by the column's span d are Markstein quotients of one reciprocal
+// (fl_rcp_mid: a span is 0, which is not divided by, or 2^-22 .. 2); the root's
 // argument lies in [1, 2], clear of the ranges that need scaling.
 //
 // 64 x 64, 60 views x 96 cells: 71 -> 11 us; 256 x 256, 256 x 256: 257 -> 36; 1024 x
@@ -133,7 +132,7 @@ __device__ __forceinline__ float fl_fan_gao_sum(const VT* __restrict__ x, const 
             const Idx col = (Idx)iu * su;
             const float xa = fl_load(x, ok1 ? col + (Idx)c1 * sv : (Idx)0), xb = fl_load(x, ok2 ? col + (Idx)c2 * sv : (Idx)0);
             const float d = vb - va, l = fl_sqrt_mid(d * d + 1.0f);
-            const float r0 = __builtin_amdgcn_rcpf(d), r = fmaf(fmaf(-d, r0, 1.0f), r0, r0);
+            const float r = fl_rcp_mid(d);
             const float wa = one ? l : sid_div(fb - va, d, r) * l, wb = sid_div(vb - fb, d, r) * l;
             t1[k] = ok1 ? wa * xa : 0.0f;
             t2[k] = ok2 ? wb * xb : 0.0f;

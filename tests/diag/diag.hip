@@ -1,7 +1,9 @@
 // diag.hip -- measurement and self-check kernels (libfl_diag.so; test and
 // profiling infrastructure, not part of libframelab_hip.so): VALU issue-peak
-// calibration for counter-based rooflines, and an exhaustive check of the
-// exact adjoint's square root against sqrtf.
+// calibration for counter-based rooflines, and exhaustive checks of the square
+// roots (fl_sqrt_mid of the exact cone adjoint's usual path and of the column
+// walk, fl_sqrt_nonneg of the whole chord routine and of the matched adjoint)
+// and of the reciprocal (fl_rcp_mid) against sqrtf and division.
 //
 // The projectors are bound by vector-ALU issue, not HBM.  To state what
 // fraction of the VALU peak they reach, the profiler's per-dispatch VALU
@@ -56,6 +58,21 @@ __global__ __launch_bounds__(256) void k_check_sqrt(unsigned long long* __restri
     if (n) atomicAdd(bad, n);
 }
 
+// Every float of [lo, hi] (bit patterns, grid-stride): KIND 0, fl_sqrt_mid against
+// sqrtf; KIND 1, fl_rcp_mid against 1.0f / d.
+template <int KIND>
+__global__ __launch_bounds__(256) void k_check_mid(uint32_t lo, uint32_t hi, unsigned long long* __restrict__ bad)
+{
+    const uint32_t stride = gridDim.x * 256u;   // 2^24
+    unsigned long long n = 0;
+    for (uint32_t p = lo + blockIdx.x * 256u + threadIdx.x; p <= hi; p += stride) {
+        const float s = __uint_as_float(p);
+        n += KIND == 0 ? __float_as_uint(fl_sqrt_mid(s)) != __float_as_uint(sqrtf(s))
+                       : __float_as_uint(fl_rcp_mid(s)) != __float_as_uint(1.0f / s);
+    }
+    if (n) atomicAdd(bad, n);
+}
+
 __global__ void k_zero_u64(unsigned long long* __restrict__ v) { *v = 0; }
 
 }  // namespace
@@ -66,6 +83,19 @@ extern "C" int fl_check_chord_sqrt(unsigned long long* d_bad, void* stream)
     if (!d_bad) return -1;
     hipLaunchKernelGGL(k_zero_u64, dim3(1), dim3(1), 0, (hipStream_t)stream, d_bad);
     hipLaunchKernelGGL(k_check_sqrt, dim3(65536), dim3(256), 0, (hipStream_t)stream, d_bad);
+    return hipGetLastError() == hipSuccess ? 0 : -2;
+}
+
+// kind 0: fl_sqrt_mid on [2^-96, 2^96); 1: fl_rcp_mid on [2^-22, 2]
+extern "C" int fl_check_mid(int kind, unsigned long long* d_bad, void* stream)
+{
+    if (!d_bad || (kind != 0 && kind != 1)) return -1;
+    hipLaunchKernelGGL(k_zero_u64, dim3(1), dim3(1), 0, (hipStream_t)stream, d_bad);
+    const auto bits = [](int e) { return (uint32_t)(e + 127) << 23; };   // of 2^e
+    if (kind == 0)
+        hipLaunchKernelGGL(k_check_mid<0>, dim3(65536), dim3(256), 0, (hipStream_t)stream, bits(-96), bits(96) - 1, d_bad);
+    else
+        hipLaunchKernelGGL(k_check_mid<1>, dim3(65536), dim3(256), 0, (hipStream_t)stream, bits(-22), bits(1), d_bad);
     return hipGetLastError() == hipSuccess ? 0 : -2;
 }
 

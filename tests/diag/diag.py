@@ -1,5 +1,5 @@
 """ctypes loader of libfl_diag.so (tests/diag/diag.hip): the VALU issue-peak
-calibration kernels and the exhaustive chord square-root check.  Test and
+calibration kernels and the exhaustive square-root and reciprocal checks.  Test and
 profiling infrastructure; the product library does not contain them."""
 from __future__ import annotations
 
@@ -19,6 +19,8 @@ def lib():
         L = C.CDLL(LIB_PATH)
         L.fl_check_chord_sqrt.restype = C.c_int
         L.fl_check_chord_sqrt.argtypes = [C.c_void_p, C.c_void_p]
+        L.fl_check_mid.restype = C.c_int
+        L.fl_check_mid.argtypes = [C.c_int, C.c_void_p, C.c_void_p]
         L.fl_calibrate_valu.restype = C.c_int
         L.fl_calibrate_valu.argtypes = [C.c_void_p, C.c_int, C.c_int, C.c_int, C.c_void_p]
         _lib = L
