@@ -220,7 +220,7 @@ def measured_traffic(kernel):
     return None
 
 
-VALU_PEAK_FP32, VALU_PEAK_INT = 0.239, 0.469   # wave-level VALU instructions per SIMD per cycle (measured)
+VALU_PEAK_FP32, VALU_PEAK_INT = 0.326, 0.469   # wave-level VALU instructions per SIMD per cycle (measured)
 SIMDS, CLOCK_HZ = 1024, 2.4e9
 
 
@@ -673,7 +673,7 @@ def main():
 
     # per-operator algorithmic bytes (per-view streaming model): nv*(Nvox*sx + Ndet*sy)
     B_op = nv * (nvox * 4 + ndet * 4)
-    dom_ms, dom_name = ((mAt, "k_adj_cone_zc<float,float,8>") if mAt >= mA
+    dom_ms, dom_name = ((mAt, "k_adj_cone_zc<float,float,8,2>") if mAt >= mA
                         else (mA, "k_fwd_cone_tr<float,float,true>"))
     achieved = B_op / (dom_ms * 1e-3) / 1e9
     roof = {"bound": "hbm", "achieved": achieved, "peak": HBM_PEAK_GBS, "unit": "GB/s",

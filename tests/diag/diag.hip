@@ -17,11 +17,16 @@
 
 namespace {
 
-// KIND 0: FP32 FMA chains; KIND 1: 32-bit integer shift/add/xor chains.
+// KIND 0: FP32 FMA chains, all operands vector registers (a scalar one makes an FMA
+// issue in over four cycles instead of three); KIND 1: 32-bit integer
+// shift/add/xor chains.
 template <int KIND>
 __global__ __launch_bounds__(256) void k_valu_peak(float* __restrict__ out, int iters, float b, float c)
 {
     const int i = blockIdx.x * 256 + threadIdx.x;
+    const float lane = 1e-9f * (float)threadIdx.x;
+    b += lane;
+    c += lane;
     float a[8];
     unsigned u[8];
 #pragma unroll
