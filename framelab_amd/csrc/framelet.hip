@@ -602,7 +602,9 @@ __global__ __launch_bounds__(256) void k_fwt2(const XT* __restrict__ u, CT* __re
     for (int b = 0; b < NF * NF; b++) fl_store(C, (size_t)b * npix + idx, w[b]);
 }
 
-// 2D synthesis, general form: the bands' neighbourhood gathered per pixel.
+// 2D synthesis, general form: the bands' neighbourhood gathered per pixel, the
+// operations and their order those of the marching form (k_iwt2m: rows outer,
+// bands of a filter inside them, then the x pass), so the same bits.
 template <int NF, int NT, typename CT, typename XT>
 __global__ __launch_bounds__(256) void k_iwt2(const CT* __restrict__ C, XT* u, int nx, int ny,
                                              int step, FlTaps T, float alpha, float beta,
@@ -612,7 +614,30 @@ __global__ __launch_bounds__(256) void k_iwt2(const CT* __restrict__ C, XT* u, i
     const size_t idx = (size_t)blockIdx.x * 256 + threadIdx.x;
     if (idx >= npix) return;
     const int x = (int)(idx % nx), y = (int)(idx / nx);
-    float v = alpha * fl_synth2<NF, NT>(C, npix, nx, ny, x, y, step, T, lp);
+    constexpr int CC = (NT - 1) / 2;
+    int xs[NT];
+    size_t row[NT];
+#pragma unroll
+    for (int k = 0; k < NT; k++) {
+        xs[k] = wrapi(x + (k - CC) * step, nx);
+        row[k] = (size_t)wrapi(y + (k - CC) * step, ny) * nx;
+    }
+    float v = 0.0f;
+    for (int i = 0; i < NF; i++) {
+        float a = 0.0f;
+#pragma unroll
+        for (int kx = 0; kx < NT; kx++) {
+            float S = 0.0f;
+#pragma unroll
+            for (int ky = 0; ky < NT; ky++)
+#pragma unroll
+                for (int j = 0; j < NF; j++)
+                    S = __builtin_fmaf(T.R[j][ky], fl_load(band_ptr(C, i + NF * j, npix, lp), row[ky] + xs[kx]), S);
+            a = __builtin_fmaf(T.R[i][kx], S, a);
+        }
+        v += a;
+    }
+    v = alpha * v;
     if (base) v = __builtin_fmaf(beta, base[idx], v);
     fl_store(u, idx, v);
 }

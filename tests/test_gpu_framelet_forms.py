@@ -96,3 +96,15 @@ def test_synthesis_2d_march_haar(gpu, level):
     u = torch.rand((1019, 1303), generator=torch.Generator(gpu).manual_seed(2), device=gpu)
     back = S.adjointTransform(S.forwardTransform(u).frameletArray)
     assert float((back - u).norm() / u.norm()) < 2e-6
+
+
+@pytest.mark.parametrize("level", [1, 2, 3])
+@pytest.mark.parametrize("frame", ["haar", "linear", "cubic"])
+def test_synthesis_2d_forms_agree(gpu, frame, level):
+    """The gather's bits are the march's: an image small enough for one form against
+    the same rows in a taller one that takes the other (Haar: 1280 x 1000 twice over;
+    the other frames march at both sizes)."""
+    from framelab_amd.framelets import FrameletSystem
+    S = FrameletSystem(2, frame, level)
+    c = torch.randn((level, S.nbands, 1000, 1280), generator=torch.Generator(gpu).manual_seed(level), device=gpu)
+    assert torch.equal(S.adjointTransform(torch.cat([c, c], 2)), S.adjointTransform(c).repeat(2, 1))
