@@ -220,7 +220,7 @@ def measured_traffic(kernel):
     return None
 
 
-VALU_PEAK_FP32, VALU_PEAK_INT = 0.326, 0.469   # wave-level VALU instructions per SIMD per cycle (measured)
+VALU_PEAK_FP32, VALU_PEAK_INT = 0.440, 0.469   # wave-level VALU instructions per SIMD per cycle (measured)
 SIMDS, CLOCK_HZ = 1024, 2.4e9
 
 

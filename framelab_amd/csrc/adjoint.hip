@@ -98,7 +98,9 @@ struct ExactLds {
 //
 // Bound by VALU issue (some 300 instructions a voxel and view at 256^3: 1.8 rows
 // of 2.3 columns at 26, and 22 more for each that some lane leaves through a z
-// face).  256^3, 360 views x 512 x 384:
+// face), at 0.25 a SIMD and cycle: of the registers 62 scalar ones, the lane
+// masks and the views' scalars, and 20 vector ones spill (84 bytes a lane).  256^3,
+// 360 views x 512 x 384:
 // 56.5 -> 48.4 ms; helix 180 x 156 x 132, 241 views x 301 x 217: 21.5 -> 8.5 ms
 // (32 rows overflowed); 64^3, 60 views: 572 -> 299 us (before: every cell's six
 // candidates, some 90 instructions).  Four waves per SIMD; three take 55.8 ms,

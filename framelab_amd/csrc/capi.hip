@@ -174,7 +174,7 @@ static int cone_ref_window_bits(const fl_geometry* g, double pa, double pb, cons
 }
 
 // Cells a pixel's shadow can meet on a fan plan's detector, for the windowed
-// adjoints (fl_fan_first_cell); 0 where they must not be used.  The windowed
+// adjoints (fl_fan_adj_tile); 0 where they must not be used.  The windowed
 // form evaluates every cell of the shadow widened by `margin` cells, which
 // holds every cell of non-zero chord or coefficient, and gives the reference's
 // sum if the reference's window (Atx_fan_mf_cpu_new.cpp:41-47) holds them too.

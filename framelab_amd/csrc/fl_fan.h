@@ -78,7 +78,7 @@ __device__ __forceinline__ float fl_fan_ray_sum(const VT* __restrict__ x, const 
 // (fl_rcp_mid: a span is 0, which is not divided by, or 2^-22 .. 2); the root's
 // argument lies in [1, 2], clear of the ranges that need scaling.
 //
-// 64 x 64, 60 views x 96 cells: 71 -> 11 us; 256 x 256, 256 x 256: 257 -> 36; 1024 x
+// 64 x 64, 60 views x 96 cells: 71 -> 9 us; 256 x 256, 256 x 256: 257 -> 36; 1024 x
 // 1024, 900 x 1000: 3.04 -> 1.47 ms (90 waves' chains of 64 columns, each
 // with a branch, a division pair, a root and a read behind one another).
 constexpr int GAO_WA = 4;
@@ -215,25 +215,9 @@ struct FlAxisIv {
     float in, out;   // entry / exit parameters of a voxel slab along one axis
 };
 
-// Entry/exit plane parameters of cell `cell` along one walk axis, with the
-// forward's plane formula ((float)i*s - o)/d.
-__device__ __forceinline__ FlAxisIv fl_slab(const SidAxis& a, int cell)
-{
-    FlAxisIv r;
-    if (!a.on) {
-        r.in = -FL_INF;
-        r.out = FL_INF;
-        return r;
-    }
-    float lo = ((float)(cell - a.nh) * a.s - a.o) / a.d;
-    float hi = ((float)(cell - a.nh + 1) * a.s - a.o) / a.d;
-    r.in = a.st > 0 ? lo : hi;
-    r.out = a.st > 0 ? hi : lo;
-    return r;
-}
-
-// As fl_slab, given rd = 1.0f / a.d: both quotients from the one reciprocal
-// (fl_div_r, bit-identical to the divisions).
+// Entry/exit plane parameters of cell `cell` along one walk axis, the forward's
+// quotients ((float)i*s - o)/d, both from rd = 1.0f / a.d (fl_div_r, bit-identical
+// to the divisions).
 __device__ __forceinline__ FlAxisIv fl_slab_r(const SidAxis& a, int cell, float rd)
 {
     FlAxisIv r;

@@ -2,9 +2,10 @@
 //
 // What a step of the walk costs is not its operations but their kind: on
 // gfx950 a wave's FP32 add, multiply and FMA, 32-bit integer add and AND, and
-// move issue in 2 to 3 cycles of its SIMD, while compares, selects, min/max,
-// shifts, conversions and three-operand integer forms take over 4 (measured,
-// throughput of independent chains).  So the walk keeps no per-step index
+// move issue in 2 to 3 cycles of its SIMD (an FMA in over 4 if an operand is a
+// scalar register), while compares, selects, min/max, shifts, conversions and
+// three-operand integer forms take over 4 (measured, throughput of independent
+// chains).  So the walk keeps no per-step index
 // arithmetic and no selects: the lanes that cross a plane update that axis
 // under the execution mask (walk_cross), and the rules that only matter at
 // rounding distance are tested once per batch of steps.

@@ -6,13 +6,16 @@
 // lies strictly between them (each axis' parameters are monotone in the
 // plane index), so that interval is exactly one element pair of the forward
 // walk.  Computing the plane parameters with the forward's float formula
-// ((float)i*s - o)/d and the length as (a_out - a_in)*|d| therefore gives the
-// forward's coefficient bit for bit, and the forward's midpoint rule decides
-// whether the walk credits v with it.  The result is the transpose of the
-// FP32 forward coefficient by coefficient (up to segments shorter than the
-// float resolution whose rounded midpoint falls in a neighbouring voxel), so
-// <Ax,y> = <x,A^T y> holds to summation rounding.  Gathers only: each thread
-// owns one voxel, no atomics, deterministic.
+// ((float)i*s - o)/d therefore gives the forward's segment a_out - a_in bit for
+// bit, |d| is the forward's too, and the forward's midpoint rule decides
+// whether the walk credits v with it (segments shorter than the float
+// resolution may have their rounded midpoint in a neighbouring voxel).  What
+// differs is the rounding of a term: where the forward adds (segment |d|) x, the
+// staged cone form adds segment (|d| y), fused with the sum; the fan and the
+// cone's general loop round segment |d| first.  The result is the transpose of
+// the FP32 forward to those roundings, so <Ax,y> = <x,A^T y> holds to
+// summation rounding.  Gathers only: a voxel's sum belongs to one thread (view
+// groups add theirs in a fixed order), no atomics, deterministic.
 //
 // No reference counterpart: the reference pairs its Siddon forward with the
 // exact-chord adjoint, whose float chords differ from the forward's lengths
@@ -62,9 +65,9 @@ struct MatchedLds {
 };
 }  // namespace
 
-// 3D, footprint-staged, z-column form: a workgroup is an 8 x 8 x 16 voxel
-// brick, and each thread of a group of four waves owns four z-adjacent voxels
-// of one (x, y) column.  Per view the group stages its footprint (MatchedLds;
+// 3D, footprint-staged, z-column form: a workgroup is a brick of 8 x 8 x 4 KZ
+// voxels (KZ = 8, or 4 in small volumes), and each thread of a group of four
+// waves owns KZ z-adjacent voxels of one (x, y) column.  Per view the group stages its footprint (MatchedLds;
 // each plane parameter the forward's IEEE quotient, formed once per group);
 // each voxel then visits the cells of its own shadow, two or three columns of a
 // row at a time.
@@ -88,9 +91,13 @@ struct MatchedLds {
 // VG groups share a brick's views between them and add their sums in group
 // order.
 //
-// Bound by VALU issue (some 120 instructions a voxel and view at 256^3: 1.8 rows
-// of 2.3 columns at 20, the rows' ranges 20, the column's slab 9, the rest the
-// tables) and by the waits between its two barriers a view.  256^3, 360 views x
+// Bound by the waits between its two barriers a view and by VALU issue: some 120
+// instructions a voxel and view at 256^3 (1.8 rows of 2.3 columns at 20, the
+// rows' ranges 20, the column's slab 9, the rest the tables), issued at 0.21 a
+// SIMD and cycle while 0.49 of the waves' cycles wait (helix 0.16 and 0.46,
+// 128^3 0.18 and 0.47, 64^3 0.16 and 0.51).  Spills, of vector and scalar
+// registers: 36 and 54 with eight slices (148 bytes a lane), 8 and 31 with four
+// (36 bytes), 4 more where dz != 1.  256^3, 360 views x
 // 512 x 384: 28.6 -> 21.4 ms; 128^3, 180 views: 2.13 -> 1.45 ms; 64^3, 60 views:
 // 276 -> 81 us; helix 180 x 156 x 132, 241 views x 301 x 217: 15.3 -> 4.0 ms
 // (before: four cell tests per pair, with a division where dz != 1, tables of

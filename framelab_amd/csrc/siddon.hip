@@ -269,6 +269,9 @@ __global__ __launch_bounds__(256) void k_to_fan_bricks(const VT* __restrict__ x,
     }
 }
 
+// Waves of FAN_WA cells x 64 / FAN_WA views.  256 x 256, 360 views x 512 cells, 82 us:
+// 0.09 instructions a SIMD and cycle with 0.94 waves there on average (2880 in
+// all), so what a call lasts is one ray's chain of steps, not issue.
 template <typename VT, typename YT, int READ>
 __global__ __launch_bounds__(256) void k_fwd_fan(const VT* __restrict__ X, YT* __restrict__ Y, FwdGeom g)
 {

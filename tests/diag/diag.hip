@@ -18,7 +18,7 @@
 namespace {
 
 // KIND 0: FP32 FMA chains, all operands vector registers (a scalar one makes an FMA
-// issue in over four cycles instead of three); KIND 1: 32-bit integer
+// issue in over four cycles instead of 2.3); KIND 1: 32-bit integer
 // shift/add/xor chains.
 template <int KIND>
 __global__ __launch_bounds__(256) void k_valu_peak(float* __restrict__ out, int iters, float b, float c)
